@@ -20,6 +20,7 @@ typedef _Float16 f16;
 typedef __bf16 bf16;
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -57,9 +58,22 @@ __device__ __forceinline__ uint16_t to_bits(float x) {
   if constexpr (std::is_same<T, f16>::value) return f2h_bits(x);
   else return f2bf_bits(x);
 }
+// two values rounded to T (bf16: one v_cvt_pk_bf16_f32, where two single conversions and the join
+// take four instructions)
 template <typename T>
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  return (uint32_t)to_bits<T>(lo) | ((uint32_t)to_bits<T>(hi) << 16);
+  if constexpr (std::is_same<T, bf16>::value)
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
+  else
+    return (uint32_t)to_bits<T>(lo) | ((uint32_t)to_bits<T>(hi) << 16);
+}
+// the exact product of an fp16 integer and an fp32 scale: with an addend (-0, which changes no
+// value) that the compiler cannot see through it is one mixed-precision FMA instead of a
+// conversion and a multiplication
+__device__ __forceinline__ float scaled_int(f16 d, float s) {
+  float none = -0.0f;
+  asm("" : "+v"(none));
+  return __builtin_fmaf((float)d, s, none);
 }
 template <typename T>
 __device__ __forceinline__ float from_bits(uint16_t b) {
@@ -120,7 +134,7 @@ __device__ __forceinline__ uint32_t deq2(uint32_t magic, const ColConst& cc) {
   if constexpr (FAST) {
     return as_u(d * as_h2(cc.sc));
   } else {
-    return pack2<T>((float)d.x * cc.scf, (float)d.y * cc.scf);
+    return pack2<T>(scaled_int(d.x, cc.scf), scaled_int(d.y, cc.scf));
   }
 }
 
