@@ -40,41 +40,30 @@ static bool decode_covers(int64_t M, int64_t G) {
 // prefill kernel's one 256-row tile per column tile keeps most CUs idle there, each tile's K
 // loop taking about 58 us at K = 4096 (measured on MI355X, K = 4096, graph replays: M = 48 / 64
 // at N = 4096 57.6 / 57.7 us against 19.5 / 24.1 us in chunks; M = 64 at N = 12288 / 24576
-// 60.6 / 62.5 against 32.9 / 38.0 us).  Above 64 rows the prefill kernel's K ranges (below)
-// are ahead of more chunks (M = 128, N = 4096: 26-27 us against 47.5 us in four chunks).
+// 60.6 / 62.5 against 32.9 / 38.0 us).  On the stream layout the middle-batch kernel (below) takes
+// these calls instead, but for forced splits.
 static bool decode_chunks(int64_t M, int64_t N, int64_t G) {
   (void)N;
   return M > 32 && M <= 64 && decode_covers(32, G);
 }
 
-// K ranges of the prefill stream kernel (split_k = 0, stream layout): where its 256 x 256 tiles
-// cover at most a third of the CUs, each tile's K loop is cut into 3 .. 8 ranges of whole stage
-// pairs (fp32 partials, summed in range order by a second launch), so that tiles x ranges
-// comes near one block per CU.  1 = no split.  Measured on MI355X (K = 4096, graph replays,
-// whole K against ranges): M = 128 .. 384 at N = 2048 .. 8192 57-64 us against 26-51 us
-// (M = 256, N = 4096: 57.9 against 26.8 us); two ranges lost (M = 384 / 512 at N = 12288 and
-// M = 2048 at N = 4096: 2-12% slower), so three is the least.
-static int prefill_splits(int64_t M, int64_t N, int64_t K, int64_t G, int32_t split_k, int32_t layout) {
-  if (split_k != 0 || layout != AWQ_LAYOUT_DECODE_STREAM || M <= 32 || decode_chunks(M, N, G)) return 1;
-  if (G <= 0 || (G & (G - 1)) != 0 || (K % 32) != 0 || (N % 8) != 0) return 1;
-  const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
-  const int64_t nst = (K + 63) / 64;
-  const int64_t cus = num_cus();
-  if (tiles * 3 > cus || nst < 12) return 1;
-  int64_t S = cus / tiles;
-  // 32 .. 63 tiles: three quarters of that (the partials' round trip grows with the ranges;
-  // M = 256 .. 512 at 32 tiles: six ranges 5-7% ahead of eight, M = 192 / 256 at 48 tiles four
-  // 2-4% ahead of five; measured on MI355X)
-  if (tiles >= 32 && tiles < 64) S = S * 3 / 4;
-  S = S > 8 ? 8 : S;
-  S = S > nst / 4 ? nst / 4 : S;  // ranges of at least four stages
-  return S < 3 ? 1 : (int)S;
-}
-// The partials go after the decode kernels' counter region, which a workspace shared between
-// calls keeps zero.
-static size_t prefill_split_bytes(int64_t M, int64_t N, int64_t K, int64_t G, int32_t split_k, int32_t layout) {
-  const int S = prefill_splits(M, N, K, G, split_k, layout);
-  return S > 1 ? kCounterBytes + (size_t)S * (size_t)M * (size_t)N * sizeof(float) : 0;
+// Whether the middle-batch kernel (awq_mid_kernel.h) serves a call on the stream layout, and its plan:
+// "auto", or a forced split_k = 1 where auto's plan keeps the whole K per block (the same bits).
+// From 25 rows on, or 17 with K <= 2048 (against the decode kernels, fp16 / bf16: K = 2048, N = 2560 M = 17
+// 9.6 / 9.4 -> 8.1 / 8.3 us, but K = 4096, N = 24576 M = 17 17.6 / 15.7 -> 17.4 / 17.2 and M = 28
+// 18.6 / 18.0 -> 16.1 / 17.5); above 64, where its estimated time is an eighth below the prefill
+// kernel's (K = 4096, graph replays, start against this kernel: M = 128 N = 4096 29.0 -> 15.3 us,
+// N = 24576 63.9 -> 33.1; M = 512 N = 4096 36.2 -> 20.9; M = 384 N = 24576 104 -> 84; at M = 512,
+// N = 24576, 100 - 108 against 103 us, the prefill kernel keeps the call).
+static bool mid_serves(int64_t M, int64_t N, int64_t K, int64_t G, int32_t split_k, int32_t layout, MidPlan* plan) {
+  if (layout != AWQ_LAYOUT_DECODE_STREAM || M <= (K <= 2048 ? 16 : 24) || split_k > 1) return false;
+  if (G < 32 || (G & (G - 1)) != 0 || (K % G) != 0 || (N % 8) != 0) return false;
+  // K <= 512 (at most one unit per share) stays with the decode kernels, which give the same bits on
+  // every layout: callers compare calls of this size across entry points
+  if (M <= 64 && (K <= 512 || !decode_covers(M <= 32 ? M : 32, G))) return false;
+  *plan = plan_mid(M, N, K, G);
+  if (split_k == 1 && plan->splits != 1) return false;
+  return M <= 64 || plan->us * 1.125 < prefill_us(M, N, K);
 }
 
 }  // namespace awq_host
@@ -159,12 +148,13 @@ int awq_w4a16_dequant(const int32_t* qweight, const void* scales, const int32_t*
                         out_dtype, (hipStream_t)stream);
 }
 
-// The decode kernels' workspace (split-K counters and partials) alone: what the allocation-free
-// entry point provides; the prefill kernel's K ranges run only where the caller's workspace
-// holds them.
+// The workspace of calls of up to 64 rows (split-K counters and partials), what the allocation-free
+// entry point provides; above 64 rows K ranges run only where the caller's workspace holds them.
 static size_t decode_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t group_size, int32_t split_k,
                                      int32_t layout) {
   if (M <= 0 || N <= 0 || K <= 0 || (N % 8) != 0 || split_k < 0) return 0;
+  MidPlan mp;
+  if (M <= 64 && mid_serves(M, N, K, group_size, split_k, layout, &mp)) return mp.ws_bytes;
   if (decode_chunks(M, N, group_size)) M = 32;  // the chunks run one after another
   if (group_size <= 0 || (K % group_size) != 0 || !decode_covers(M, group_size)) return 0;
   if (layout == AWQ_LAYOUT_DECODE_NARROW) return 0;  // the narrow kernel does not split K
@@ -182,9 +172,9 @@ static size_t decode_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t gr
 size_t awq_w4a16_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t group_size,
                                       int32_t split_k, int32_t layout) {
   if (M <= 0 || N <= 0 || K <= 0 || (N % 8) != 0 || split_k < 0) return 0;
-  const size_t pre = (group_size > 0 && (K % group_size) == 0) ? prefill_split_bytes(M, N, K, group_size, split_k, layout) : 0;
-  const size_t dec = decode_workspace_bytes(M, N, K, group_size, split_k, layout);
-  return pre > dec ? pre : dec;
+  MidPlan mp;
+  if (mid_serves(M, N, K, group_size, split_k, layout, &mp)) return mp.ws_bytes;
+  return decode_workspace_bytes(M, N, K, group_size, split_k, layout);
 }
 
 }  // extern "C"
@@ -243,6 +233,16 @@ static int gemm_impl(const void* a, int64_t lda, const int32_t* qweight, const v
     if (!launch_decode_narrow(ga, zp, act_dtype, scale_dtype, st)) return AWQ_ERR_UNSUPPORTED;
     return launch_status();
   }
+  MidPlan mp;
+  if (rows <= 1 && mid_serves(M, N, K, group_size, split_k, layout, &mp)) {
+    const bool held = workspace && workspace_bytes >= mp.ws_bytes && !(((uintptr_t)workspace) & 15);
+    if (mp.ws_bytes == 0 || held) {
+      ga.partial = mp.ws_bytes ? (float*)((char*)workspace + kCounterBytes) : nullptr;
+      launch_mid(ga, mp, act_dtype, scale_dtype, st);
+      return launch_status();
+    }
+    if (M <= 64) return AWQ_ERR_WORKSPACE;
+  }
   if (decode_covers(M, group_size)) {
     const DecodeMode mode = decode_mode(layout, act_dtype, scale_dtype);
     const DecodePlan sp = plan_decode(M, N, K, group_size, split_k, mode);
@@ -272,13 +272,6 @@ static int gemm_impl(const void* a, int64_t lda, const int32_t* qweight, const v
   }
   if ((K % 32) != 0) return AWQ_ERR_SHAPE;
   if (layout == AWQ_LAYOUT_DECODE_STREAM) {
-    // K ranges where the workspace holds their fp32 partials (else the whole K per tile)
-    const int S = rows <= 1 ? prefill_splits(M, N, K, group_size, split_k, layout) : 1;
-    if (S > 1 && workspace && !(((uintptr_t)workspace) & 15) &&
-        workspace_bytes >= kCounterBytes + (size_t)S * (size_t)M * (size_t)N * sizeof(float)) {
-      ga.partial = (float*)((char*)workspace + kCounterBytes);
-      ga.ksplit = S;
-    }
     if (!launch_prefill_stream(ga, zp, act_dtype, scale_dtype, st)) return AWQ_ERR_UNSUPPORTED;
   } else if (!launch_prefill(ga, seq, zp, act_dtype, scale_dtype, st)) {
     return AWQ_ERR_UNSUPPORTED;
@@ -305,8 +298,8 @@ int awq_w4a16_gemm_noalloc(const void* a, int64_t lda, const int32_t* qweight, c
                            int32_t scale_dtype, int32_t bias_dtype, void* stream) {
   if (M < 0 || N < 0 || K <= 0 || group_size <= 0 || split_k < 0) return AWQ_ERR_SHAPE;
   if (M == 0 || N == 0) return AWQ_OK;
-  // the decode kernels' split-K needs only: prefill calls get no workspace here, so each of
-  // their tiles takes the whole K
+  // up to 64 rows only: larger calls get no workspace here, so their plans with K ranges give way to the
+  // prefill kernel, whose tiles take the whole K
   const size_t need = decode_workspace_bytes(M, N, K, group_size, split_k, layout);
   if (need > kNoallocScratchBytes) return AWQ_ERR_WORKSPACE;  // beyond the fixed scratch
   void* ws = nullptr;

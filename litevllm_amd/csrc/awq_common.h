@@ -240,7 +240,7 @@ struct GemmArgs {
   const uint32_t* qz;
   const void* bias;
   uint16_t* c;
-  float* partial;   // decode: [tiles, max_contrib, M, tile columns] fp32
+  float* partial;   // decode: [tiles, max_contrib, M, tile columns] fp32; middle batches: awq_mid_kernel.h
   int* counters;    // decode: [tiles], zero on entry and on exit
   int64_t lda, ldc;
   int M, N, K, G;
@@ -257,9 +257,6 @@ struct GemmArgs {
   // decode kernels only: > 1 = a row-exact launch (awq_w4a16_gemm_rows_exact) of that many grid
   // rows, M = 1: grid row y computes row y of the call as a lone M = 1 call would (row_slice)
   int rows;
-  // prefill stream kernel only: > 1 = split K into that many ranges of whole stage pairs, each
-  // writing its fp32 sums to partial[split][M][N], summed in split order by a second launch
-  int ksplit;
 };
 
 // Block coordinates of a stream-kernel decode launch: x = the block of the M = 1 plan (nblocks

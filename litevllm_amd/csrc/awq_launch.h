@@ -61,6 +61,19 @@ bool launch_prefill(const awq::GemmArgs& a, bool seq, bool zp, int act, int sdt,
 // Prefill GEMM on the decode stream layout (awq_prefill.hip): M > 32, K % 32 == 0.
 bool launch_prefill_stream(const awq::GemmArgs& a, bool zp, int act, int sdt, hipStream_t st);
 
+// Middle-batch GEMM on the decode stream layout (awq_mid_kernel.h): column tiles x K ranges of
+// `per` units x row tiles of 16 mt rows; ws_bytes covers the ranges' fp32 partials, us is the
+// plan's estimated time.
+struct MidPlan {
+  int mt, tiles, splits, row_tiles, per;
+  size_t ws_bytes;
+  double us;
+};
+MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int64_t G);
+void launch_mid(const awq::GemmArgs& a, const MidPlan& m, int act, int sdt, hipStream_t st);
+// Estimated time of the prefill stream kernel's launches for a call.
+double prefill_us(int64_t M, int64_t N, int64_t K);
+
 // Standalone dequant and repack.
 int launch_dequant(const int32_t* qweight, const void* scales, const int32_t* qzeros, void* out,
                    int64_t rows, int64_t cols, int32_t group_size, int32_t layout,

@@ -1,0 +1,90 @@
+"""The middle-batch GEMM (17 rows to a few hundred, ``awq_mid_kernel.h``) through ``ops.gemm``, at the edges
+of its tiles: row tiles of 16 to 128 rows, a partial column tile, K that ends inside a stage, K ranges,
+shares without work.  Every output within one ulp (of max(|y|, 1)) of the float64 product with the weights
+that the path multiplies: unrounded up to 64 rows, rounded once to the activation dtype above; bitwise
+the same on a second call."""
+import numpy as np
+import pytest
+import torch
+
+from kernel_paths import decode_serves
+from oracle import awq_oracle as O
+from oracle.gen import make_awq_problem
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _expected(p, x, sc, G, zp, half, bias=None):
+    M, N = x.shape[0], p["qweight"].shape[1] * 8
+    out = "float32" if decode_serves(M, N, G) else half
+    w = O.dequant_awq(p["qweight"], sc.float().numpy(), p["qzeros"] if zp else None, G, out_dtype=out, zero_point=zp)
+    w = O.bf16_bits_to_f32(w) if out == "bfloat16" else w
+    y = x.double().numpy() @ w.astype(np.float64)
+    return y if bias is None else y + bias.double().numpy()
+
+
+@pytest.mark.parametrize("M,K,N,G", [
+    (17, 2048, 136, 64), (25, 1024, 8, 128), (32, 4096, 264, 128), (33, 544, 520, 32), (48, 1088, 1000, 64),
+    (49, 2080, 264, 32), (64, 3072, 1024, 128), (65, 512, 2056, 128), (80, 96, 24, 32), (97, 1088, 136, 64),
+    (128, 2080, 520, 32), (129, 2048, 1024, 256), (200, 1408, 392, 128), (400, 1024, 264, 64)])
+@pytest.mark.parametrize("act,sdt,zp", [(torch.float16, torch.float16, True), (torch.float16, torch.float16, False),
+                                        (torch.float16, torch.bfloat16, True), (torch.bfloat16, torch.float16, True),
+                                        (torch.bfloat16, torch.bfloat16, False)])
+def test_mid_batch_vs_oracle(M, K, N, G, act, sdt, zp):
+    from litevllm_amd import ops
+    print(f"mid batch M={M} K={K} N={N} G={G} {act} scales={sdt} zp={zp}", flush=True)
+    p = make_awq_problem(M=M, K=K, N=N, group_size=G, seed=M + K + N, with_bias=True)
+    x, sc = torch.from_numpy(p["x"]).to(act), torch.from_numpy(p["scales"]).to(sdt)
+    b = torch.from_numpy(p["bias"])
+    qz = torch.from_numpy(p["qzeros"]).to(DEV) if zp else None
+    args = (x.to(DEV), torch.from_numpy(p["qweight"]).to(DEV), sc.to(DEV), qz, G)
+    y, y2 = (ops.gemm(*args, bias=b.to(DEV), layout="autoawq") for _ in range(2))
+    assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
+    ye = _expected(p, x, sc, G, zp, "float16" if act == torch.float16 else "bfloat16", b)
+    ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(ye), 1.0))) - (10 if act == torch.float16 else 7))
+    err = np.abs(y.double().cpu().numpy() - ye) / ulp
+    assert err.max() <= 1.0, float(err.max())
+
+
+@pytest.mark.parametrize("M", [40, 200])
+def test_mid_batch_strides_capture_and_scratch(M):
+    """Strided rows in and out, replays of a captured call, the allocation-free entry point, and a
+    workspace that does not hold the plan's K ranges (refused up to 64 rows, the prefill kernel above)."""
+    from litevllm_amd import _lib as L
+    from litevllm_amd import ops
+    K, N, G = 2048, 512, 128
+    p = make_awq_problem(M=M, K=K, N=N, group_size=G, seed=M)
+    t = {k: torch.from_numpy(v).to(DEV) for k, v in p.items() if isinstance(v, np.ndarray)}
+    call = lambda x, out=None: ops.gemm(x, t["qweight"], t["scales"], t["qzeros"], G, layout="autoawq", out=out)
+    y = call(t["x"])
+    xb = torch.zeros((M, K + 64), dtype=torch.float16, device=DEV)
+    xb[:, :K] = t["x"]
+    ob = torch.full((M, N + 64), 7.0, dtype=torch.float16, device=DEV)
+    call(xb[:, :K], ob[:, :N])
+    assert torch.equal(ob[:, :N], y) and bool((ob[:, N:] == 7.0).all())
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        yg = call(t["x"])
+    for _ in range(3):
+        yg.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(yg, call(t["x"]))
+    lib = L.load()
+    qk = ops.pack_decode_stream(t["qweight"])
+    ws = int(lib.awq_w4a16_gemm_workspace_bytes(M, N, K, G, 0, L.LAYOUT_DECODE_STREAM))
+    assert ws > 65536  # K ranges
+    out = torch.empty_like(y)
+    head = (t["x"].data_ptr(), K, qk.data_ptr(), t["scales"].data_ptr(), t["qzeros"].data_ptr(), None, out.data_ptr(), N, M, N, K,
+            G, 0, L.LAYOUT_DECODE_STREAM, L.DTYPE_F16, L.DTYPE_F16, L.DTYPE_NONE)
+    st = int(torch.cuda.current_stream().cuda_stream)
+    small = torch.zeros(ws - 4, dtype=torch.uint8, device=DEV)
+    rc = lib.awq_w4a16_gemm(*head, small.data_ptr(), ws - 4, st)
+    assert rc == (L.ERR_WORKSPACE if M <= 64 else 0)
+    assert lib.awq_w4a16_gemm_noalloc(*head, st) == 0
+    if M <= 64:
+        assert torch.equal(out, y)
+    else:  # the prefill kernel: the same products in another order
+        assert float((out.float() - y.float()).abs().max()) <= 2 * float(y.float().abs().max()) * 2.0 ** -10
