@@ -238,6 +238,7 @@ static int gemm_impl(const void* a, int64_t lda, const int32_t* qweight, const v
     const bool held = workspace && workspace_bytes >= mp.ws_bytes && !(((uintptr_t)workspace) & 15);
     if (mp.ws_bytes == 0 || held) {
       ga.partial = mp.ws_bytes ? (float*)((char*)workspace + kCounterBytes) : nullptr;
+      ga.counters = (int*)workspace;
       launch_mid(ga, mp, act_dtype, scale_dtype, st);
       return launch_status();
     }

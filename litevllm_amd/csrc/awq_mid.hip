@@ -10,9 +10,10 @@ using namespace awq;
 // One block per CU; a block's time on MI355X is 2 us + 0.35 us per 16 rows outside its K loop
 // and 0.21 us + 0.08 us per 16 rows for each k-step of a share (128 k of the block), which
 // reproduces N = 24576, K = 4096 at one round of blocks (M = 32 / 48 / 64 / 80 / 96 / 128: 18.2 / 20.2 /
-// 22.3 / 24.5 / 28.7 / 33.1 us) to 5%.  K ranges add the reduction launch (3 us) and the
-// partials' round trip (about 6 TB/s): M = 128, N = K = 4096 takes 15.3 us as 4 ranges x 2 row
-// tiles of 64 rows and 21.0 us as 8 ranges x 1 of 128.  Up to 64 rows there is one row tile;
+// 22.3 / 24.5 / 28.7 / 33.1 us) to 5%.  K ranges add, up to 64 rows,
+// the hand-off (1.5 us) and one block's reading of its tile's partials (8 KB per range and 16 rows at
+// about 100 bytes a ns), above them the reduction launch (3 us) and the partials' round trip (about 6
+// TB/s).  Up to 64 rows there is one row tile;
 // above, row tiles of 64 .. 128 rows: the plan with the least estimated time.
 MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int64_t G) {
   const int64_t tiles = cdiv(N, 128), cus = num_cus();
@@ -32,7 +33,7 @@ MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int64_t G) {
       if (M <= 64 && parts > kMidPartialMax) break;
       const double rounds = (double)cdiv(tiles * m.row_tiles * m.splits, cus);
       const double ksteps = (double)cdiv(m.per, kMidShares) * (double)(unit / 32);
-      m.us = 2.0 + rounds * (2.0 + 0.35 * m.mt + ksteps * (0.21 + 0.08 * m.mt)) + (m.splits > 1 ? 3.0 + (double)parts / 3e6 : 0.0);
+      m.us = 2.0 + rounds * (2.0 + 0.35 * m.mt + ksteps * (0.21 + 0.08 * m.mt)) + (m.splits == 1 ? 0.0 : M <= 64 ? 1.5 + 0.08 * m.mt * m.splits : 3.0 + (double)parts / 3e6);
       m.ws_bytes = parts ? kCounterBytes + parts : 0;
       if (best.mt == 0 || m.us < best.us) best = m;
     }
@@ -53,7 +54,7 @@ void launch_mid(const GemmArgs& a, const MidPlan& m, int act, int sdt, hipStream
   else if (act == AWQ_DTYPE_F16 && sdt == AWQ_DTYPE_F16) launch_unr<f16, true>(a, m.mt, wk, st);
   else if (act == AWQ_DTYPE_F16) launch_unr<f16, false>(a, m.mt, wk, st);
   else launch_unr<bf16, false>(a, m.mt, wk, st);
-  if (m.splits > 1) {
+  if (a.M > 64 && m.splits > 1) {
     const dim3 grid((unsigned)cdiv(cdiv(a.M, 4) * m.tiles, 4));
     if (act == AWQ_DTYPE_F16) hipLaunchKernelGGL((mid_reduce_kernel<f16>), grid, dim3(256), 0, st, a, wk);
     else hipLaunchKernelGGL((mid_reduce_kernel<bf16>), grid, dim3(256), 0, st, a, wk);

@@ -20,7 +20,8 @@
 //    ones per row tile, taken off per group.  Otherwise they enter as (q - z) * s rounded once, the
 //    prefill kernels'.
 //  * The shares' sums meet in LDS in share order; with one K range the block writes its outputs,
-//    with several it writes fp32 partials, which a second launch adds in range order.
+//    with several it writes fp32 partials, which the tile's last block (UNR) or a second launch adds
+//    in range order.
 //  * The blocks of a column tile's row tiles are dispatched together on one XCD and read the
 //    tile's weights through its L2.
 //  * What bounds it: short calls, fixed costs (M = 64, N = K = 4096, 15.2 us: 1.3 us to the first operands,
@@ -163,14 +164,14 @@ __global__ void __launch_bounds__(512, 2) mid_kernel(const GemmArgs p, const Mid
   };
   // activations: a DMA instruction fills 8 rows of a stage, lane l row l / 8, slot l % 8, which holds
   // chunk slot ^ swz(row) (an operand read, 16 rows at 4 chunks, then covers all 64 banks); wave e of
-  // a share issues its half of them.  Rows past M read as zero (the descriptor's range check).
+  // a share issues its half of them.  Rows past M repeat the last one and are never stored.
   auto swz = [](int row) { return (row ^ (row >> 3)) & 7; };
   uint32_t a_voff[ND];
 #pragma unroll
   for (int i = 0; i < ND; ++i) {
     const int row = 8 * (e * ND + i) + (lane >> 3);
     const int kc = (lane & 7) ^ swz(row & 15);
-    a_voff[i] = ((uint32_t)(m0 + row) * (uint32_t)p.lda + (uint32_t)(kc * 8)) * 2u;
+    a_voff[i] = ((uint32_t)min(m0 + row, p.M - 1) * (uint32_t)p.lda + (uint32_t)(kc * 8)) * 2u;
   }
   // activation instruction i of stage s into ring slot `aslot`
   auto req_a = [&](int s, int aslot, int i) {
@@ -393,7 +394,32 @@ __global__ void __launch_bounds__(512, 2) mid_kernel(const GemmArgs p, const Mid
   // ---- the shares' sums meet: [share][row quad][column] x 4 rows; column 8 r + 2 P + e of the tile at
   // 64 e + 16 P + r.  Each output is summed in share order ----
   constexpr int RQ = RPASS / 4;
-  const int rq_total = (p.M + 3) >> 2;
+  const int rq_total = (p.M + 3) >> 2, rq0 = m0 >> 2;
+  // partials: [range][row quad][column tile][128 columns] x 4 rows
+  const __amdgpu_buffer_rsrc_t prs = make_rsrc(p.partial, (uint32_t)wk.splits * (uint32_t)rq_total * (uint32_t)wk.tiles * 2048u);
+  const uint32_t pbase = (uint32_t)((split * rq_total + rq0) * wk.tiles + t) * 2048u;
+  // four rows of columns 8 r + 2 P and the next -> the block's 16-bit output tile in LDS; whole rows of it
+  // then leave in 16-byte pieces
+  auto stage_out = [&](int rq, int pr, const f32x4 (&o)[2]) {
+    __attribute__((address_space(3))) uint32_t* outl = (__attribute__((address_space(3))) uint32_t*)(uintptr_t)(lds0 + RED);
+    const int P = pr >> 4, c = pr & 15, col = t * 128 + 8 * c + 2 * P;
+    float b0 = 0.f, b1 = 0.f;
+    if (p.bias && col < p.N) {
+      b0 = load_bias(p.bias, p.bias_dtype, col);
+      b1 = load_bias(p.bias, p.bias_dtype, col + 1);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) outl[(4 * rq + v) * 64 + 4 * c + P] = pack2<T>(o[0][v] + b0, o[1][v] + b1);
+  };
+  auto write_out = [&](int mp, int nq) {
+    __syncthreads();
+    for (int i = tid; i < nq * 64; i += 512) {  // (row, word)
+      const int row = i >> 4, c = i & 15, grow = m0 + 16 * mp + row, gword = t * 16 + c;
+      const u32x4 v = rd(lds0 + (uint32_t)(RED + row * 256 + c * 16));
+      if (grow < p.M && gword < NW) *(u32x4*)(p.c + (int64_t)grow * p.ldc + 8 * gword) = v;
+    }
+    __syncthreads();
+  };
 #pragma unroll
   for (int mp = 0; mp < MT; mp += 4) {
     __syncthreads();
@@ -406,9 +432,8 @@ __global__ void __launch_bounds__(512, 2) mid_kernel(const GemmArgs p, const Mid
             UNR ? tot[UNR ? mt : 0][P] : acc[mt][P];
     __syncthreads();
     const int nq = (ROWS - 16 * mp < RPASS ? ROWS - 16 * mp : RPASS) / 4;
-    __attribute__((address_space(3))) uint32_t* outl = (__attribute__((address_space(3))) uint32_t*)(uintptr_t)(lds0 + RED);
     for (int i = tid; i < nq * 64; i += 512) {  // (row quad, P, r): columns 8 r + 2 P, 8 r + 2 P + 1
-      const int rq = i >> 6, pr = i & 63, P = pr >> 4, c = pr & 15;
+      const int rq = i >> 6, pr = i & 63;
       f32x4 o[2];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
@@ -418,33 +443,63 @@ __global__ void __launch_bounds__(512, 2) mid_kernel(const GemmArgs p, const Mid
         for (int w = 1; w < kMidShares; ++w)
           o[h] += *(__attribute__((address_space(3))) const f32x4*)(uintptr_t)(ad + (uint32_t)(w * RQ * 2048));
       }
-      if (wk.splits > 1) {
-        const int rqg = (m0 + 16 * mp) / 4 + rq;
-        if (rqg < rq_total) {
-          f32x4* dst = (f32x4*)p.partial + ((size_t)(split * rq_total + rqg) * (size_t)wk.tiles + (size_t)t) * 128;
-          dst[pr] = o[0];
-          dst[64 + pr] = o[1];
-        }
-      } else {
-        const int col = t * 128 + 8 * c + 2 * P;
-        float b0 = 0.f, b1 = 0.f;
-        if (p.bias && col < p.N) {
-          b0 = load_bias(p.bias, p.bias_dtype, col);
-          b1 = load_bias(p.bias, p.bias_dtype, col + 1);
-        }
-#pragma unroll
-        for (int v = 0; v < 4; ++v) outl[(4 * rq + v) * 64 + 4 * c + P] = pack2<T>(o[0][v] + b0, o[1][v] + b1);
+      if (wk.splits == 1) {
+        stage_out(rq, pr, o);
+      } else if (rq0 + 4 * mp + rq < rq_total) {
+        const int off = (int)pbase + ((4 * mp + rq) * wk.tiles * 128 + pr) * 16;
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o[0]), prs, off, 0, kDeviceCoherent);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o[1]), prs, off + 1024, 0, kDeviceCoherent);
       }
     }
-    if (wk.splits == 1) {
-      __syncthreads();
-      for (int i = tid; i < nq * 64; i += 512) {  // (row, word)
-        const int row = i >> 4, c = i & 15, grow = m0 + 16 * mp + row, gword = t * 16 + c;
-        const u32x4 v = rd(lds0 + (uint32_t)(RED + row * 256 + c * 16));
-        if (grow < p.M && gword < NW) *(u32x4*)(p.c + (int64_t)grow * p.ldc + 8 * gword) = v;
-      }
-    }
+    if (wk.splits == 1) write_out(mp, nq);
   }
+  if (!UNR || wk.splits == 1) return;
+
+  // ---- K ranges, up to 64 rows: the block that arrives last at its (column tile, row tile) adds the ranges' partials in
+  // range order.  The count is an agent-scope release after the block's (device-scope) stores and the
+  // last block takes an acquire fence, as in the decode kernels.  Against a second launch over the
+  // partials, N = K = 4096: M = 32 11.7 -> 10.5 us, M = 57 14.6 -> 13.3; above 64 rows, where one block
+  // would read up to 400 KB and the tile's other row tiles wait, the second launch stays ahead
+  // (mid_reduce_kernel; four projections of 200 rows, twice: 270 against 289 us) ----
+  __attribute__((address_space(3))) int* s_last = (__attribute__((address_space(3))) int*)(uintptr_t)lds0;  // the sums are done with
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  int* counter = p.counters + rt * wk.tiles + t;
+  if (tid == 0) {
+    *s_last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT) == wk.splits - 1;
+    if (*s_last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  }
+  __syncthreads();
+  if (!*s_last) return;
+  const uint32_t plane = (uint32_t)rq_total * (uint32_t)wk.tiles * 2048u;  // bytes between ranges
+#pragma unroll
+  for (int mp = 0; mp < MT; mp += 4) {
+    const int nq = (ROWS - 16 * mp < RPASS ? ROWS - 16 * mp : RPASS) / 4;
+    for (int i = tid; i < nq * 64; i += 512) {
+      const int rq = i >> 6, pr = i & 63;
+      if (rq0 + 4 * mp + rq >= rq_total) continue;
+      const uint32_t off = (uint32_t)(((rq0 + 4 * mp + rq) * wk.tiles + t) * 128 + pr) * 16u;
+      f32x4 o[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+      for (int s0 = 0; s0 < wk.splits; s0 += 4) {  // four ranges' loads in flight; those past the last read zero
+        f32x4 v[4][2];
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            v[s][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                    prs, s0 + s < wk.splits ? (int)(off + (uint32_t)(s0 + s) * plane + 1024u * h) : (int)0x80000000,
+                                                    0, kDeviceCoherent));
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          o[0] += v[s][0];
+          o[1] += v[s][1];
+        }
+      }
+      stage_out(rq, pr, o);
+    }
+    write_out(mp, nq);
+  }
+  if (tid == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // c[4 rq + v][...] = round(sum over splits, in split order, of the partials + bias): a wave per (row
