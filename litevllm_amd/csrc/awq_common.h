@@ -67,6 +67,20 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
   else
     return (uint32_t)to_bits<T>(lo) | ((uint32_t)to_bits<T>(hi) << 16);
 }
+// an output value (or two) of a kernel computing in T; via_bf16 (fp16 kernels): the fp16 result
+// converted to bf16, two roundings, as a store of it into a bf16 tensor gives
+template <typename T>
+__device__ __forceinline__ uint16_t out_bits(float x, bool via_bf16) {
+  if constexpr (std::is_same<T, f16>::value)
+    if (via_bf16) return f2bf_bits((float)(f16)x);
+  return to_bits<T>(x);
+}
+template <typename T>
+__device__ __forceinline__ uint32_t out_pack2(float lo, float hi, bool via_bf16) {
+  if constexpr (std::is_same<T, f16>::value)
+    if (via_bf16) return pack2<bf16>((float)(f16)lo, (float)(f16)hi);
+  return pack2<T>(lo, hi);
+}
 // the exact product of an fp16 integer and an fp32 scale: with an addend (-0, which changes no
 // value) that the compiler cannot see through it is one mixed-precision FMA instead of a
 // conversion and a multiplication
@@ -250,10 +264,12 @@ struct GemmArgs {
   // 64 t + j (j < 64, below n_out) is act(gate) * up of tile t's columns j and 64 + j.
   int gate_act, n_out;
   // narrow decode kernel only: non-NULL = normalise the staged activation rows first
-  // (RMSNorm prologue, fp16 rows; norm_w [K] fp16, or bf16 when norm_bf16)
+  // (RMSNorm prologue; rows fp16, or bf16 when c_bf16; norm_w [K] fp16, or bf16 when norm_bf16)
   const uint16_t* norm_w;
   float eps;
   int norm_bf16;
+  // fp16 kernels: the fp16 result is stored converted to bf16 (RMSNorm + GEMM of a bf16 tensor)
+  int c_bf16;
   // decode kernels only: > 1 = a row-exact launch (awq_w4a16_gemm_rows_exact) of that many grid
   // rows, M = 1: grid row y computes row y of the call as a lone M = 1 call would (row_slice)
   int rows;

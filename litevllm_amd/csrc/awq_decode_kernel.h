@@ -407,7 +407,7 @@ decode_kn_kernel(const GemmArgs p_in, const DecodeWork wk) {
     if (S == 1) {
       if (col < ncols) {
         if (p.bias) sum += load_bias(p.bias, p.bias_dtype, t * 128 + col);
-        p.c[(int64_t)m * p.ldc + t * 128 + col] = to_bits<T>(sum);
+        p.c[(int64_t)m * p.ldc + t * 128 + col] = out_bits<T>(sum, p.c_bf16);
       }
     } else {
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, sum), prs, (int)(pbase + 4u * (uint32_t)o), 0,
@@ -486,7 +486,7 @@ decode_kn_kernel(const GemmArgs p_in, const DecodeWork wk) {
       sum[0] += load_bias(p.bias, p.bias_dtype, col);
       sum[1] += load_bias(p.bias, p.bias_dtype, col + 1);
     }
-    *(uint32_t*)(p.c + (int64_t)m * p.ldc + col) = pack2<T>(sum[0], sum[1]);
+    *(uint32_t*)(p.c + (int64_t)m * p.ldc + col) = out_pack2<T>(sum[0], sum[1], p.c_bf16);
   }
   if (tid == 0) __hip_atomic_store(&p.counters[t], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

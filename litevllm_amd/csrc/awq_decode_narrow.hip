@@ -43,7 +43,7 @@ __host__ __device__ inline NarrowLds narrow_lds(int nwv, int mrows, int ngroups,
   return l;
 }
 
-// RMSNorm prologue (rmsnorm_awq_fused.py:108-131) for one fp16 row staged by XL: the row
+// RMSNorm prologue (rmsnorm_awq_fused.py:108-131) for one fp16 or bf16 row staged by XL: the row
 // arrives in registers instead of by DMA -- lane tid holds the 16-byte pieces pc = tid,
 // tid + NT, .. (at most kNormCols of them) with the matching 16 bytes of the norm weights.
 // The sum of squares (exact squares added in fp64: lanes by DPP, then the waves through
@@ -51,9 +51,11 @@ __host__ __device__ inline NarrowLds narrow_lds(int nwv, int mrows, int ngroups,
 // element is written to the staged row in LDS as fp16((x * rrms) * norm_w).
 constexpr int kNormCols = 6;
 
-template <int NT>
+template <int NT, bool XBF>  // XBF: a bf16 row
 struct NormRow {
   u32x4 x[kNormCols], g[kNormCols];
+
+  static __device__ __forceinline__ float value(uint16_t b) { return XBF ? bf_bits2f(b) : h_bits2f(b); }
 
   __device__ __forceinline__ void load(const GemmArgs& p, int tid) {
     const int kp = p.K >> 3;
@@ -80,7 +82,7 @@ struct NormRow {
         double s0 = 0.0, s1 = 0.0;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const double lo = h_bits2f((uint16_t)(x[u][j] & 0xFFFF)), hi = h_bits2f((uint16_t)(x[u][j] >> 16));
+          const double lo = value((uint16_t)(x[u][j] & 0xFFFF)), hi = value((uint16_t)(x[u][j] >> 16));
           s0 += lo * lo;
           s1 += hi * hi;
         }
@@ -104,8 +106,8 @@ struct NormRow {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const uint16_t glo = (uint16_t)(g[u][j] & 0xFFFF), ghi = (uint16_t)(g[u][j] >> 16);
-          const float lo = fp32_rounded((h_bits2f((uint16_t)(x[u][j] & 0xFFFF)) * rr) * (nbf ? bf_bits2f(glo) : h_bits2f(glo)));
-          const float hi = fp32_rounded((h_bits2f((uint16_t)(x[u][j] >> 16)) * rr) * (nbf ? bf_bits2f(ghi) : h_bits2f(ghi)));
+          const float lo = fp32_rounded((value((uint16_t)(x[u][j] & 0xFFFF)) * rr) * (nbf ? bf_bits2f(glo) : h_bits2f(glo)));
+          const float hi = fp32_rounded((value((uint16_t)(x[u][j] >> 16)) * rr) * (nbf ? bf_bits2f(ghi) : h_bits2f(ghi)));
           o[j] = (uint32_t)f2h_bits(lo) | ((uint32_t)f2h_bits(hi) << 16);
         }
         *(u32x4*)(xs + 8 * pc) = o;
@@ -120,7 +122,7 @@ struct NormRow {
 // and are never read back); otherwise each quad's activations come with its weights, per lane.
 // NORM (one fp16 row staged by XL, K / 8 <= kNormCols * NWV * 64): the row comes through
 // registers and is staged normalised (RMSNorm prologue) before the first k-step.
-template <int MT, int NWV, int SPG, bool ZP, typename T, bool SBF, bool ONE, bool XL, bool NORM = false>
+template <int MT, int NWV, int SPG, bool ZP, typename T, bool SBF, bool ONE, bool XL, bool NORM = false, bool XBF = false>
 __global__ void __launch_bounds__(NWV * 64) decode_narrow_kernel(const GemmArgs p_in, int tiles) {
   static_assert(!ONE || MT == 1, "");
   static_assert(!XL || MT == 1, "");
@@ -220,7 +222,7 @@ __global__ void __launch_bounds__(NWV * 64) decode_narrow_kernel(const GemmArgs 
       }
     }
   }
-  NormRow<NWV * 64> npc;
+  NormRow<NWV * 64, XBF> npc;
   if constexpr (NORM) npc.load(p, tid);
   // every load of this wave has landed (the ring's first quads with it: they were issued
   // together); the barrier then covers every wave's DMA (with NORM the prologue's first)
@@ -335,7 +337,7 @@ __global__ void __launch_bounds__(NWV * 64) decode_narrow_kernel(const GemmArgs 
     const int oc = t * 16 + c;
     if (oc < p.N) {
       if (p.bias) sum += load_bias(p.bias, p.bias_dtype, oc);
-      p.c[(int64_t)m * p.ldc + oc] = to_bits<T>(sum);
+      p.c[(int64_t)m * p.ldc + oc] = out_bits<T>(sum, p.c_bf16);
     }
   }
 }
@@ -392,7 +394,7 @@ int launch_pack_decode_narrow(const int32_t* qweight_kn, int32_t* out, int64_t K
 // in 64 KiB, or in the CU's 160 KiB when the tiles fit the CUs once (one block per CU anyway)
 constexpr uint32_t kNarrowLdsMax = 65536, kNarrowLdsMaxOne = 163840;
 
-template <int MT, bool ZP, typename T, bool SBF, bool ONE, bool XL, bool NORM = false>
+template <int MT, bool ZP, typename T, bool SBF, bool ONE, bool XL, bool NORM = false, bool XBF = false>
 static bool launch_narrow_t(const GemmArgs& a, hipStream_t st) {
   const int tiles = (int)cdiv(a.N, 16);
   const int spg = a.G / 32;
@@ -402,7 +404,7 @@ static bool launch_narrow_t(const GemmArgs& a, hipStream_t st) {
   if (L.total > (tiles <= num_cus() ? kNarrowLdsMaxOne : kNarrowLdsMax)) return false;
   if (NORM && a.K / 8 > (int64_t)kNormCols * nwv * 64) return false;
 #define AWQ_NARROW_L(NWV, SPG_) \
-  hipLaunchKernelGGL((decode_narrow_kernel<MT, NWV, SPG_, ZP, T, SBF, ONE, XL, NORM>), grid, dim3((NWV) * 64), L.total, st, a, tiles)
+  hipLaunchKernelGGL((decode_narrow_kernel<MT, NWV, SPG_, ZP, T, SBF, ONE, XL, NORM, XBF>), grid, dim3((NWV) * 64), L.total, st, a, tiles)
   if (nwv == 16) {
     if (spg == 4) AWQ_NARROW_L(16, 4);
     else if (spg == 2) AWQ_NARROW_L(16, 2);
@@ -424,12 +426,15 @@ static bool launch_narrow_m(const GemmArgs& a, hipStream_t st) {
   return launch_narrow_t<1, ZP, T, SBF, true, true>(a, st) || launch_narrow_t<1, ZP, T, SBF, true, false>(a, st);
 }
 
-// The RMSNorm prologue variant: one fp16 row, fp16 scales, the row staged in LDS (false when
+// The RMSNorm prologue variant: one fp16 or bf16 row, fp16 scales, the row staged in LDS (false when
 // it does not fit; the caller then normalises in a launch of its own).  Only M = 1: for 2 .. 4
 // rows the prologue measured no faster on MI355X than the separate row-norm launch (K = 4096,
 // N = 6144: 11.0 us against 10.2 us of kernels plus the launch gap).
 bool launch_decode_narrow_norm(const GemmArgs& a, bool zp, hipStream_t st) {
   if (a.M != 1 || !a.norm_w) return false;
+  if (a.c_bf16)  // a bf16 row
+    return zp ? launch_narrow_t<1, true, f16, false, true, true, true, true>(a, st)
+              : launch_narrow_t<1, false, f16, false, true, true, true, true>(a, st);
   return zp ? launch_narrow_t<1, true, f16, false, true, true, true>(a, st)
             : launch_narrow_t<1, false, f16, false, true, true, true>(a, st);
 }

@@ -263,7 +263,7 @@ __global__ void __launch_bounds__(128 * NWN, 2) prefill_kn_kernel(const GemmArgs
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int row = wave_m * WM + mt * 16 + 4 * q + v;
-        cl[row * BN + c_chunk(row, cc >> 3) * 8 + (cc & 7)] = to_bits<T>(acc[mt][nt][v] + bv);
+        cl[row * BN + c_chunk(row, cc >> 3) * 8 + (cc & 7)] = out_bits<T>(acc[mt][nt][v] + bv, p.c_bf16);
       }
     }
   }

@@ -409,7 +409,7 @@ __global__ void __launch_bounds__(512, 2) mid_kernel(const GemmArgs p, const Mid
       b1 = load_bias(p.bias, p.bias_dtype, col + 1);
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) outl[(4 * rq + v) * 64 + 4 * c + P] = pack2<T>(o[0][v] + b0, o[1][v] + b1);
+    for (int v = 0; v < 4; ++v) outl[(4 * rq + v) * 64 + 4 * c + P] = out_pack2<T>(o[0][v] + b0, o[1][v] + b1, p.c_bf16);
   };
   auto write_out = [&](int mp, int nq) {
     __syncthreads();
@@ -529,7 +529,7 @@ __global__ void __launch_bounds__(256) mid_reduce_kernel(const GemmArgs p, const
       b1 = load_bias(p.bias, p.bias_dtype, col + 1);
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) outl[wave][v * 64 + 4 * c + P] = pack2<T>(o[0][v] + b0, o[1][v] + b1);
+    for (int v = 0; v < 4; ++v) outl[wave][v * 64 + 4 * c + P] = out_pack2<T>(o[0][v] + b0, o[1][v] + b1, p.c_bf16);
   }
   __syncthreads();
   const int grow = 4 * rq + P, gword = t * 16 + c;

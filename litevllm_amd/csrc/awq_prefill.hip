@@ -360,7 +360,7 @@ __global__ void __launch_bounds__(128 * NWN, 2) prefill_stream_kernel(const Gemm
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = 128 * wm + 32 * mt + 8 * (r >> 2) + 4 * lh + (r & 3);
-        cl[row * BN + c_chunk(row, cc >> 3) * 8 + (cc & 7)] = to_bits<T>(acc[mt][nt][r] + bv);
+        cl[row * BN + c_chunk(row, cc >> 3) * 8 + (cc & 7)] = out_bits<T>(acc[mt][nt][r] + bv, p.c_bf16);
       }
     }
   }

@@ -1,0 +1,41 @@
+"""The fused RMSNorm + GEMM of bf16 rows: every GEMM kernel's epilogue converts its fp16 result to bf16, so
+the call equals, bit for bit, the fp16 GEMM of the normalised rows converted afterwards.  The row norm at the
+edges of its register form (2048 elements a column, up to 8 columns) against the oracle, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import awq_oracle as O
+from oracle.gen import make_awq_problem
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+@pytest.mark.parametrize("M,K,N,G,kw", [
+    (1, 1024, 512, 128, {}), (1, 1024, 512, 128, {"decode_layout": "stream"}), (8, 4096, 1024, 128, {"decode_layout": "stream"}),
+    (16, 1024, 264, 64, {}), (24, 512, 136, 32, {"decode_layout": "narrow"}), (40, 2048, 264, 128, {}), (100, 4096, 520, 128, {}),
+    (300, 256, 65536, 128, {}), (64, 512, 264, 128, {"decode_stream": False}), (130, 512, 264, 128, {"decode_stream": False})])
+def test_bf16_rows_equal_converted_fp16_result(M, K, N, G, kw):
+    from litevllm_amd import ops
+    print(f"rmsnorm bf16 M={M} K={K} N={N} G={G} {kw}", flush=True)
+    t = {k: torch.from_numpy(v).to(DEV) for k, v in make_awq_problem(M=M, K=K, N=N, group_size=G, seed=M + N).items()
+         if isinstance(v, np.ndarray)}
+    x = t["x"].to(torch.bfloat16)
+    nw = (1 + 0.3 * torch.randn(K, generator=torch.Generator().manual_seed(K))).to(torch.bfloat16).to(DEV)
+    w = (t["qweight"], t["scales"], t["qzeros"], G)
+    y = ops.rmsnorm_gemm(x, nw, 1e-6, *w, layout="autoawq", **kw)
+    # the bf16 call's weight copy: the layout rule sees bf16 activations
+    if not kw and M <= 32:
+        kw = {"decode_layout": "narrow" if ops._narrow_fits(M, N, K, 0, True) else "stream"}
+    xn = ops.rmsnorm(x, nw, 1e-6)
+    assert torch.equal(y, ops.gemm(xn, *w, layout="autoawq", **kw).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("K", [8, 2048, 2056, 8192, 8200, 16384, 16392])
+def test_rows_at_column_edges(K):
+    from litevllm_amd import ops
+    g = torch.Generator().manual_seed(K)
+    x, nw = torch.randn(3, K, generator=g).half(), (1 + 0.3 * torch.randn(K, generator=g)).half()
+    got = ops.rmsnorm(x.to(DEV), nw.to(DEV), 1e-6).cpu().numpy()
+    assert np.array_equal(got.view(np.uint16), O.rmsnorm_rows(x.float().numpy(), nw.float().numpy(), 1e-6).view(np.uint16))
