@@ -502,10 +502,10 @@ using namespace awq;
 // Activation slices up to this many bytes per block are staged in LDS (M == 1, stream layout).
 constexpr uint32_t kDecodeXlMax = 49152;
 
-template <int MT, bool SEQ, bool ZP, typename T, bool SBF, bool STREAM, bool ONE, bool XL>
+template <int MT, bool SEQ, bool ZP, typename T, bool SBF, bool STREAM, bool ONE, bool XL, int NWV = ONE ? 16 : 8>
 inline void launch_x(const GemmArgs& a, const DecodePlan& s, uint32_t shmem, hipStream_t st) {
   const DecodeWork wk{s.tiles, s.ksteps, s.splits, s.per};
-  constexpr int NWV = ONE ? 16 : 8, OCC = ONE ? 4 : 2;
+  constexpr int OCC = ONE ? 4 : 2;
   const dim3 grid((unsigned)(s.blocks * (a.rows > 1 ? a.rows : 1))), block(NWV * 64);
   const int spg = a.G / 32;
   if (spg == 4)
@@ -520,8 +520,23 @@ template <int MT, bool SEQ, bool ZP, typename T, bool SBF, bool STREAM, bool ONE
 inline void launch_t(const GemmArgs& a, const DecodePlan& s, hipStream_t st) {
   if constexpr (ONE && STREAM) {
     const uint32_t xbytes = (uint32_t)((s.per + 15) / 16) * 1024u;  // whole DMA instructions
+    // more whole-K tiles than CUs: blocks of 8 waves, two per CU, so that a round and a part round of 16-wave
+    // blocks run at once (K = 4096, N = 34816 / 43008 / 65536 / 131072: 21.6 -> 19.4 / 22.5 -> 20.4 /
+    // 28.4 -> 26.0 / 50.7 -> 47.2 us; gate and up of K = 5376, I = 21504, group 32, 32.0 -> 29.8)
+    if (xbytes <= kDecodeXlMax && s.splits == 1 && s.tiles > num_cus()) {
+      launch_x<MT, SEQ, ZP, T, SBF, STREAM, ONE, true, 8>(a, s, xbytes, st);
+      return;
+    }
     if (xbytes <= kDecodeXlMax) {
       launch_x<MT, SEQ, ZP, T, SBF, STREAM, ONE, true>(a, s, xbytes, st);
+      return;
+    }
+  }
+  if constexpr (!ONE && STREAM) {
+    // the same with blocks of 4 waves, up to two tiles per CU (K = 4096, M = 8: N = 34816 23.6 -> 21.0 us, N =
+    // 65536 28.8 -> 26.4; at N = 81920 they trail, 37.5 -> 38.2)
+    if (s.splits == 1 && s.tiles > num_cus() && s.tiles <= 2 * num_cus()) {
+      launch_x<MT, SEQ, ZP, T, SBF, STREAM, ONE, false, 4>(a, s, 0, st);
       return;
     }
   }
