@@ -62,9 +62,9 @@ extern "C" {
  * AWQ_LAYOUT_DECODE_STREAM : an AUTOAWQ qweight re-ordered by awq_w4a16_pack_decode_stream so
  *                      that the decode kernel reads it as contiguous 2 KiB runs; qzeros and
  *                      scales stay in the AUTOAWQ layout.  Accepted by awq_w4a16_gemm for every
- *                      M (K % 32 == 0): the decode kernel serves M <= 32 with group sizes
- *                      32/64/128 (and 32-row chunks of it up to M = 64), the prefill
- *                      kernel the rest, so one copy serves both.
+ *                      M (K % 32 == 0): the decode kernel serves up to 16 or 24 rows with group
+ *                      sizes 32/64/128, the middle-batch kernel up to a few hundred, the
+ *                      prefill kernel the rest, so one copy serves all.
  * AWQ_LAYOUT_DECODE_NARROW : an AUTOAWQ qweight re-ordered by awq_w4a16_pack_decode_narrow
  *                      into 16-column tiles cut along K into quads of four 32-row k-steps
  *                      (KQ = ceil(K / 128) quads per tile; k-steps past K are zero): the run of
@@ -117,8 +117,9 @@ int awq_w4a16_dequant(const int32_t* qweight, const void* scales, const int32_t*
 
 /* Workspace bytes awq_w4a16_gemm needs for these arguments (0 if none).  The workspace
  * starts with a fixed 64 KiB region of per-tile arrival counters followed by fp32 split-K
- * partials (the decode kernels', or the prefill kernel's K ranges: [ranges][M][N]; a prefill
- * call given less than that runs its whole K per tile).  The counter region must be zero the first time a workspace is used; every
+ * partials (the decode kernels', or the middle-batch kernel's K ranges; a call of the latter given
+ * less than that runs on the decode kernels up to 64 rows, if it holds their partials, and on the
+ * prefill kernel above).  The counter region must be zero the first time a workspace is used; every
  * call leaves it zero again, so a workspace allocated zeroed once can be reused by later
  * calls of any shape on the same stream.  Two calls that may run concurrently must not
  * share a workspace. */
@@ -126,10 +127,10 @@ size_t awq_w4a16_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t g
                                       int32_t split_k, int32_t layout);
 
 /* C[M, N] = A[M, K] . dequant(W)^T (+ bias), products accumulated in fp32, one rounding to
- * act_dtype at the end.  M <= 32 with group_size 32, 64 or 128 (the decode kernel; calls up to
- * M = 64 run as 32-row chunks on it, one launch each, in order on the stream): the weights
+ * act_dtype at the end.  M <= 64 with group_size 32, 64 or 128 (the decode kernels, above 32 rows in
+ * 32-row chunks, or the middle-batch kernel on the stream layout): the weights
  * enter unrounded, (q - z) * s in fp32 -- the reference's M = 1
- * formulation, awq_fused_gemm.py:1966-1971.  Otherwise (the prefill kernel): W rounded once to act_dtype,
+ * formulation, awq_fused_gemm.py:1966-1971.  Otherwise: W rounded once to act_dtype,
  * as awq_w4a16_dequant computes it (the reference's tl.dot branch, 1973-1976).
  *   a: [M, K] act_dtype (F16 or BF16), row stride lda (elements).
  *   layout: AUTOAWQ or KN_SEQ (qweight [K, N/8]), DECODE_STREAM (any M) or DECODE_NARROW

@@ -243,7 +243,8 @@ static int gemm_impl(const void* a, int64_t lda, const int32_t* qweight, const v
       launch_mid(ga, mp, act_dtype, scale_dtype, st);
       return launch_status();
     }
-    if (M <= 64) return AWQ_ERR_WORKSPACE;
+    // too small a workspace for the plan's K ranges: the decode kernels up to 64 rows, where it holds theirs
+    // (K < 1536: none), the prefill kernel above
   }
   if (decode_covers(M, group_size)) {
     const DecodeMode mode = decode_mode(layout, act_dtype, scale_dtype);

@@ -50,7 +50,8 @@ def test_mid_batch_vs_oracle(M, K, N, G, act, sdt, zp):
 @pytest.mark.parametrize("M", [40, 200])
 def test_mid_batch_strides_capture_and_scratch(M):
     """Strided rows in and out, replays of a captured call, the allocation-free entry point, and a
-    workspace that does not hold the plan's K ranges (refused up to 64 rows, the prefill kernel above)."""
+    workspace that does not hold the plan's K ranges (the decode kernels up to 64 rows where it holds theirs,
+    the prefill kernel above)."""
     from litevllm_amd import _lib as L
     from litevllm_amd import ops
     K, N, G = 2048, 512, 128
@@ -81,10 +82,33 @@ def test_mid_batch_strides_capture_and_scratch(M):
             G, 0, L.LAYOUT_DECODE_STREAM, L.DTYPE_F16, L.DTYPE_F16, L.DTYPE_NONE)
     st = int(torch.cuda.current_stream().cuda_stream)
     small = torch.zeros(ws - 4, dtype=torch.uint8, device=DEV)
-    rc = lib.awq_w4a16_gemm(*head, small.data_ptr(), ws - 4, st)
-    assert rc == (L.ERR_WORKSPACE if M <= 64 else 0)
+    assert lib.awq_w4a16_gemm(*head, small.data_ptr(), ws - 4, st) == 0
+    # other kernels, the same products in another order
+    assert float((out.float() - y.float()).abs().max()) <= 2 * float(y.float().abs().max()) * 2.0 ** -10
+    # without one: 64 rows and K = 2048 need ranges on the decode kernels too
+    assert lib.awq_w4a16_gemm(*head, None, 0, st) == (L.ERR_WORKSPACE if M <= 64 else 0)
     assert lib.awq_w4a16_gemm_noalloc(*head, st) == 0
     if M <= 64:
         assert torch.equal(out, y)
     else:  # the prefill kernel: the same products in another order
         assert float((out.float() - y.float()).abs().max()) <= 2 * float(y.float().abs().max()) * 2.0 ** -10
+
+
+@pytest.mark.parametrize("M", [32, 57])
+def test_mid_batch_without_workspace_where_decode_needs_none(M):
+    """K = 1504: the plan cuts K, the decode kernels' plan does not, so a call without a workspace runs."""
+    from litevllm_amd import _lib as L
+    from litevllm_amd import ops
+    K, N, G = 1504, 512, 32
+    p = make_awq_problem(M=M, K=K, N=N, group_size=G, seed=M)
+    t = {k: torch.from_numpy(v).to(DEV) for k, v in p.items() if isinstance(v, np.ndarray)}
+    lib, qk = L.load(), ops.pack_decode_stream(t["qweight"])
+    assert int(lib.awq_w4a16_gemm_workspace_bytes(M, N, K, G, 0, L.LAYOUT_DECODE_STREAM)) > 65536
+    out = torch.empty((M, N), dtype=torch.float16, device=DEV)
+    rc = lib.awq_w4a16_gemm(t["x"].data_ptr(), K, qk.data_ptr(), t["scales"].data_ptr(), t["qzeros"].data_ptr(), None, out.data_ptr(),
+                            N, M, N, K, G, 0, L.LAYOUT_DECODE_STREAM, L.DTYPE_F16, L.DTYPE_F16, L.DTYPE_NONE, None, 0,
+                            int(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    ye = _expected(p, t["x"].cpu(), t["scales"].cpu(), G, True, "float16")
+    ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(ye), 1.0))) - 10)
+    assert (np.abs(out.double().cpu().numpy() - ye) / ulp).max() <= 1.0
