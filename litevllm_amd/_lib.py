@@ -102,6 +102,8 @@ class AWQKernelError(RuntimeError):
 def load(path: str | None = None) -> ctypes.CDLL:
     """Load (once) and return the library; raises ``OSError`` if it is not built."""
     global _lib
+    if path is None and _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None and path is None:
             return _lib
