@@ -387,6 +387,9 @@ using namespace awq;
 double prefill_us(int64_t M, int64_t N, int64_t K) {
   const int64_t tm = cdiv(M, kPSBM), tn4 = cdiv(N, 256), cus = num_cus();
   if (tm * tn4 * 4 < cus * 3) return 2.0 + 0.017 * (double)K * (double)cdiv(tm * cdiv(N, 128), cus);
+  // the two launches of a row-tile count that does not divide the CUs are left out: the middle-batch kernel
+  // is ahead of them where they would decide (M = 700, N = 24576 170 against 185 us; M = 1500, N = 12288
+  // 171 against 183)
   const int64_t full = cus % tm == 0 ? tn4 / (cus / tm) * (cus / tm) : 0, rest = cdiv(N - full * 256, 128);
   if (full > 0 && rest > 0 && tm * rest <= cus)
     return 2.0 + (double)K * (0.026 * (double)(tm * full / cus) + 0.017);
@@ -423,16 +426,15 @@ static void launch_ps(const GemmArgs& a, int sbf, int log2g, hipStream_t st) {
   // Whole rounds of 256-column blocks, then a part round of them as 128-column blocks in a
   // second launch, where those fill the chip once: the part round runs at twice the blocks
   // for half the work each instead of leaving CUs idle (M = 2048, N = 12288: 384 blocks, 1.5
-  // rounds).
-  if (cus % tm == 0) {
-    const int per_round = cus / tm;  // 256-column tiles per round of blocks
-    const int full = tn4 / per_round * per_round;
-    const int rest = (int)cdiv(a.N - full * 256, 128);
-    if (full > 0 && rest > 0 && (int64_t)tm * rest <= cus) {
-      wide(full, 0);
-      narrow(rest, full * 256);
-      return;
-    }
+  // rounds).  Also at row-tile counts that do not divide the CUs (K = 4096, one part round of
+  // 256-column blocks against this: M = 1500 N = 24576 316 -> 301 us, N = 22016 314 -> 298; M = 1700
+  // N = 28672 427 -> 406; M = 1200 N = 28672 313 -> 296).
+  const int64_t full = (int64_t)tm * tn4 / cus * cus / tm;  // 256-column tiles of the whole rounds
+  const int64_t rest = cdiv(a.N - full * 256, 128);
+  if (full > 0 && rest > 0 && tm * rest <= cus) {
+    wide((int)full, 0);
+    narrow((int)rest, (int)full * 256);
+    return;
   }
   wide(tn4, 0);
 }
