@@ -15,10 +15,12 @@
 //    own VALU work between its MFMAs is nearly free up to three instructions each, and adds in
 //    full anywhere else.
 //  * UNR (M <= 64): the weights enter the MFMA as exact integers and each group's sum is scaled once in
-//    fp32, the decode kernels' unrounded formulation: q - z for fp16, 128 + q for bf16 (whose exact q - z
-//    would take three conversions a pair), with (128 + z) times the activation sums, an MFMA against
-//    ones per row tile, taken off per group.  Otherwise they enter as (q - z) * s rounded once, the
-//    prefill kernels'.
+//    fp32, the decode kernels' unrounded formulation: q - z for fp16, and for bf16 in groups of 32; 128 + q
+//    for bf16 in larger groups (exact q - z takes three conversions a pair), with (128 + z) times the
+//    activation sums, an MFMA against ones per row tile, taken off per group.  The bias costs precision
+//    where one activation is far above the others (1e4 among N(0, 1), group 32: 2.2 bf16 ulps against 0.5)
+//    and turns an infinite one into NaN in every column, so it is taken only where the decode kernels'
+//    two-tile form takes it.  Otherwise they enter as (q - z) * s rounded once, the prefill kernels'.
 //  * The shares' sums meet in LDS in share order; with one K range the block writes its outputs,
 //    with several it writes fp32 partials, which the tile's last block (UNR) or a second launch adds
 //    in range order.
@@ -185,7 +187,7 @@ __global__ void __launch_bounds__(512, 2) mid_kernel(const GemmArgs p, const Mid
     lds_dma16(ars, lds0 + (uint32_t)(aslot * STAGE + part * ABYTES + (e * ND + i) * 1024), vo, (uint32_t)(k * 2));
   };
 
-  constexpr bool BIAS = UNR && std::is_same<T, bf16>::value;
+  constexpr bool BIAS = UNR && std::is_same<T, bf16>::value && GK != 32;
   f32x4 acc[MT][4];
   f32x4 ax[BIAS ? MT : 1];  // the group's activation sums
   f32x4 tot[UNR ? MT : 1][4];
@@ -241,7 +243,8 @@ __global__ void __launch_bounds__(512, 2) mid_kernel(const GemmArgs p, const Mid
       }
       const f16x2 d = as_h2(magic_bits<P>(w[u], mk)) - zz;  // exact q - z
       if constexpr (UNR) {
-        v[u] = as_u(d);
+        if constexpr (std::is_same<T, f16>::value) v[u] = as_u(d);
+        else v[u] = pack2<T>((float)d.x, (float)d.y);
       } else if constexpr (FAST) {
         const f16x2 sh = as_h2(sc2[P >> 1]);
         const f16x2 ss = (P & 1) ? __builtin_shufflevector(sh, sh, 1, 1) : __builtin_shufflevector(sh, sh, 0, 0);

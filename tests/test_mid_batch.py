@@ -112,3 +112,25 @@ def test_mid_batch_without_workspace_where_decode_needs_none(M):
     ye = _expected(p, t["x"].cpu(), t["scales"].cpu(), G, True, "float16")
     ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(ye), 1.0))) - 10)
     assert (np.abs(out.double().cpu().numpy() - ye) / ulp).max() <= 1.0
+
+
+@pytest.mark.parametrize("M,K,N", [(20, 1024, 264), (25, 1056, 136), (32, 2080, 264), (40, 1024, 520), (64, 2048, 1000)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_outlier_and_infinite_activations_in_groups_of_32(M, K, N, dt):
+    """Groups of 32: the operands are q - z themselves, so an activation far above its row's others adds nothing
+    where q == z, and an infinite one gives +-inf wherever q != z and NaN (0 * inf) only where q == z."""
+    from litevllm_amd import ops
+    print(f"outliers M={M} K={K} N={N} {dt}", flush=True)
+    G = 32
+    p = make_awq_problem(M=M, K=K, N=N, group_size=G, seed=M + K + N)
+    x = torch.from_numpy(p["x"]).to(dt)
+    x[::2, 100] = 2e4
+    x[1, 40], x[3, 41] = float("inf"), float("-inf")
+    w = tuple(torch.from_numpy(p[k]).to(DEV) for k in ("qweight", "scales", "qzeros")) + (G,)
+    y = ops.gemm(x.to(DEV), *w, layout="autoawq").double().cpu().numpy()
+    with np.errstate(invalid="ignore"):  # 0 * inf
+        ye = _expected(p, x, torch.from_numpy(p["scales"]), G, True, "float16")
+    fin = np.isfinite(ye)
+    assert np.array_equal(y[~fin], ye[~fin], equal_nan=True)
+    ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(ye[fin]), 1.0))) - (10 if dt == torch.float16 else 7))
+    assert (np.abs(y[fin] - ye[fin]) / ulp).max() <= 1.0
