@@ -327,7 +327,7 @@ int awq_w4a16_moe(const void* x, int64_t ldx, const void* topk_ids, int32_t ids_
 int awq_w4a16_gate_up_interleave(const void* gate, const void* up, void* out, int64_t rows, int64_t cols,
                                  int32_t elem_bytes, int32_t half_tile, void* stream);
 
-/* Workspace of awq_w4a16_gate_up_act: that of awq_w4a16_gemm for the interleaved matrix,
+/* Workspace of awq_w4a16_gate_up_act: the decode kernels' split-K plan for the interleaved matrix,
  * N = 2 * ceil(I / 64) * 64 (same zeroing rule); 0 for DECODE_NARROW. */
 size_t awq_w4a16_gate_up_workspace_bytes(int64_t M, int64_t I, int64_t K, int32_t group_size,
                                          int32_t split_k, int32_t layout);

@@ -148,13 +148,10 @@ int awq_w4a16_dequant(const int32_t* qweight, const void* scales, const int32_t*
                         out_dtype, (hipStream_t)stream);
 }
 
-// The workspace of calls of up to 64 rows (split-K counters and partials), what the allocation-free
-// entry point provides; above 64 rows K ranges run only where the caller's workspace holds them.
+// The decode kernels' workspace (split-K counters and partials) alone.
 static size_t decode_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t group_size, int32_t split_k,
                                      int32_t layout) {
   if (M <= 0 || N <= 0 || K <= 0 || (N % 8) != 0 || split_k < 0) return 0;
-  MidPlan mp;
-  if (M <= 64 && mid_serves(M, N, K, group_size, split_k, layout, &mp)) return mp.ws_bytes;
   if (decode_chunks(M, N, group_size)) M = 32;  // the chunks run one after another
   if (group_size <= 0 || (K % group_size) != 0 || !decode_covers(M, group_size)) return 0;
   if (layout == AWQ_LAYOUT_DECODE_NARROW) return 0;  // the narrow kernel does not split K
@@ -167,6 +164,15 @@ static size_t decode_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t gr
     ws = b > ws ? b : ws;
   }
   return ws;
+}
+
+// What the allocation-free entry point provides: a GEMM call's workspace up to 64 rows; above, K ranges run
+// only where the caller's workspace holds them.
+static size_t small_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t group_size, int32_t split_k,
+                                    int32_t layout) {
+  MidPlan mp;
+  if (M <= 64 && mid_serves(M, N, K, group_size, split_k, layout, &mp)) return mp.ws_bytes;
+  return decode_workspace_bytes(M, N, K, group_size, split_k, layout);
 }
 
 size_t awq_w4a16_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t group_size,
@@ -303,7 +309,7 @@ int awq_w4a16_gemm_noalloc(const void* a, int64_t lda, const int32_t* qweight, c
   if (M == 0 || N == 0) return AWQ_OK;
   // up to 64 rows only: larger calls get no workspace here, so their plans with K ranges give way to the
   // prefill kernel, whose tiles take the whole K
-  const size_t need = decode_workspace_bytes(M, N, K, group_size, split_k, layout);
+  const size_t need = small_workspace_bytes(M, N, K, group_size, split_k, layout);
   if (need > kNoallocScratchBytes) return AWQ_ERR_WORKSPACE;  // beyond the fixed scratch
   void* ws = nullptr;
   if (need > 0) {
@@ -508,7 +514,9 @@ int awq_w4a16_gate_up_interleave(const void* gate, const void* up, void* out, in
 size_t awq_w4a16_gate_up_workspace_bytes(int64_t M, int64_t I, int64_t K, int32_t group_size,
                                          int32_t split_k, int32_t layout) {
   if (I <= 0 || layout == AWQ_LAYOUT_DECODE_NARROW) return 0;
-  return awq_w4a16_gemm_workspace_bytes(M, 2 * cdiv(I, 64) * 64, K, group_size, split_k, layout);
+  // the gated launch is the decode kernels' at every M it takes, also where the GEMM of the interleaved
+  // matrix would run on the middle-batch kernel, whose plan may need less
+  return decode_workspace_bytes(M, 2 * cdiv(I, 64) * 64, K, group_size, split_k, layout);
 }
 
 int awq_w4a16_gate_up_act(const void* x, int64_t ldx, const int32_t* qweight, const void* scales,

@@ -283,3 +283,33 @@ def test_gate_up_interleave_layout():
     assert torch.equal(out[:, :64], s[:, :64]) and torch.equal(out[:, 64:128], 2 * s[:, :64])
     assert torch.equal(out[:, 128:164], s[:, 64:]) and torch.equal(out[:, 192:228], 2 * s[:, 64:])
     assert not out[:, 164:192].any() and not out[:, 228:].any()
+
+
+# ---------------------------------------------------------------- workspace of the gated launch
+# the decode plan cuts K into more ranges here than the GEMM of the interleaved matrix does
+MANY_RANGES = [(25, 2560, 6176), (32, 2560, 6176)]
+
+
+@pytest.mark.parametrize("M,n,k", MANY_RANGES + [(17, 1024, 2048), (32, 4096, 4096), (32, 64, 8192)])
+def test_gate_up_workspace_holds_the_decode_plan(M, n, k):
+    """The size query answers for the decode plan, which runs the gated launch at every M it takes: counters and
+    S ranges of fp32 partials."""
+    from litevllm_amd import _lib as L
+    from litevllm_amd import ops
+    N = 2 * (-(-n // 64)) * 64
+    S = ops._auto_splits(M, N, k)
+    assert S > 1
+    ws = int(L.load().awq_w4a16_gate_up_workspace_bytes(M, n, k, 32, 0, L.LAYOUT_DECODE_STREAM))
+    assert ws >= 65536 + S * M * N * 4, (ws, S)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,n,k", MANY_RANGES)
+def test_gate_up_act_many_ranges(M, n, k):
+    from litevllm_amd import ops
+    print(f"gate_up_act many ranges M={M} n={n} k={k}", flush=True)
+    pair = _pair(n, k, seed=M, sdt=torch.float16)
+    (qg, sg), (qu, su) = pair
+    x = torch.randn(M, k, dtype=torch.float16, generator=torch.Generator().manual_seed(M))
+    y = ops.gate_up_act(x.to(DEV), qg.to(DEV), qu.to(DEV), sg.to(DEV), su.to(DEV), 32, activation="silu")
+    _check(y, _exact(x, pair, 32, "silu"), torch.float16, (M, n, k))
