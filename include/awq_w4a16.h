@@ -369,9 +369,10 @@ size_t awq_w4a16_rmsnorm_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, i
  * awq_w4a16_rmsnorm into the workspace, then awq_w4a16_gemm on the fp16 rows (any layout it
  * takes, no bias), C rounded to fp16; for BF16 activations that fp16 result is converted to
  * bf16 (round to nearest even), as the reference's store into a bf16 output does
- * (rmsnorm_awq_fused.py:170-175).  C: [M, N] act_dtype, row stride ldc.  Three launches at
- * most, all on `stream`; one for the DECODE_NARROW layout with F16 activations and scales and
- * M = 1, whose kernel normalises the row it stages (when the row fits its LDS). */
+ * (rmsnorm_awq_fused.py:170-175), in the GEMM's epilogue.  C: [M, N] act_dtype, row stride ldc; it may
+ * lie over x or norm_w.  The row norm's launch, then the GEMM's, all on `stream`; one launch for the
+ * DECODE_NARROW layout with F16 scales and M = 1, whose kernel normalises the row it stages (when the
+ * row fits its LDS and C lies apart from x and norm_w). */
 int awq_w4a16_rmsnorm_gemm(const void* x, int64_t ldx, const void* norm_w, float eps,
                            const int32_t* qweight, const void* scales, const int32_t* qzeros, void* c,
                            int64_t ldc, int64_t M, int64_t N, int64_t K, int32_t group_size, int32_t split_k,

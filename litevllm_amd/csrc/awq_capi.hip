@@ -592,6 +592,11 @@ int awq_w4a16_rmsnorm(const void* x, int64_t ldx, const void* norm_w, float eps,
   return launch_rmsnorm_rows(x, ldx, norm_w, eps, xn, ldxn, M, K, act_dtype, norm_dtype, (hipStream_t)stream);
 }
 
+static bool apart(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
+  const uintptr_t ua = (uintptr_t)a, ub = (uintptr_t)b;
+  return ua + a_bytes <= ub || ub + b_bytes <= ua;
+}
+
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 size_t awq_w4a16_rmsnorm_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t group_size,
@@ -629,8 +634,10 @@ int awq_w4a16_rmsnorm_gemm(const void* x, int64_t ldx, const void* norm_w, float
   if (layout == AWQ_LAYOUT_DECODE_NARROW && scale_dtype == AWQ_DTYPE_F16 && M == 1 &&
       decode_covers(M, group_size) && (K % 32) == 0 && decode_narrow_bytes(K, N) <= 0x7FFFFFFFLL &&
       M * ldx * 2 <= 0x7FFFFFFFLL && !(((uintptr_t)qweight) & 15) && !(((uintptr_t)scales) & 15) &&
-      !(((uintptr_t)norm_w) & 15)) {
-    // one launch: the narrow kernel normalises its staged rows itself
+      !(((uintptr_t)norm_w) & 15) && apart(c, (size_t)N * 2, x, (size_t)K * 2) &&
+      apart(c, (size_t)N * 2, norm_w, (size_t)K * 2)) {
+    // one launch: the narrow kernel normalises its staged rows itself.  Every block reads the whole row and
+    // the norm weights, so an output that lies over them takes the two launches below
     GemmArgs ga{};
     ga.a = (const uint16_t*)x;
     ga.qw = (const uint32_t*)qweight;

@@ -39,3 +39,23 @@ def test_rows_at_column_edges(K):
     x, nw = torch.randn(3, K, generator=g).half(), (1 + 0.3 * torch.randn(K, generator=g)).half()
     got = ops.rmsnorm(x.to(DEV), nw.to(DEV), 1e-6).cpu().numpy()
     assert np.array_equal(got.view(np.uint16), O.rmsnorm_rows(x.float().numpy(), nw.float().numpy(), 1e-6).view(np.uint16))
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,off", [(1, 0), (1, 2048), (8, 0)])
+def test_output_over_the_input_rows(M, off, dt):
+    """An output that lies over x, wholly or from its middle on: the values of a call whose output lies apart (the
+    narrow kernel's blocks read the row while others store, so such a call normalises in a launch of its own)."""
+    from litevllm_amd import ops
+    K = N = 4096
+    print(f"rmsnorm in place M={M} off={off} {dt}", flush=True)
+    p = make_awq_problem(M=M, K=K, N=N, group_size=128, seed=5)
+    w = tuple(torch.from_numpy(p[k]).to(DEV) for k in ("qweight", "scales", "qzeros")) + (128,)
+    nw = (1 + 0.3 * torch.randn(K, generator=torch.Generator().manual_seed(K))).half().to(DEV)
+    buf = torch.zeros(M * K + off, dtype=dt, device=DEV)
+    x, out = buf[: M * K].view(M, K), buf[off:].view(M, N)
+    x.copy_(torch.from_numpy(p["x"]))
+    want = ops.rmsnorm_gemm(x, nw, 1e-6, *w, layout="autoawq", decode_layout="narrow")
+    assert ops.rmsnorm_gemm(x, nw, 1e-6, *w, layout="autoawq", decode_layout="narrow", out=out).data_ptr() == out.data_ptr()
+    # the narrow kernel's own norm and the row-norm launch give the same rows
+    assert torch.equal(out, want)
