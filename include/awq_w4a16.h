@@ -360,8 +360,9 @@ int awq_w4a16_rmsnorm(const void* x, int64_t ldx, const void* norm_w, float eps,
 
 /* Workspace of awq_w4a16_rmsnorm_gemm: awq_w4a16_gemm's (same zeroing rule, at offset 0, and
  * never less than its 64 KiB counter region, so one workspace can serve both functions), then
- * the normalised rows [M, K] fp16, then for BF16 activations the fp16 product [M, N]; each
- * part starts on a 256-byte boundary and the workspace itself on one. */
+ * the normalised rows [M, K] fp16; each part starts on a 256-byte boundary and the workspace
+ * itself on one.  For BF16 activations the answer includes 2 M N bytes that earlier versions
+ * used; the call itself needs only the answer for F16. */
 size_t awq_w4a16_rmsnorm_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t group_size,
                                               int32_t split_k, int32_t layout, int32_t act_dtype);
 

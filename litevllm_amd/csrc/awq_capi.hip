@@ -599,16 +599,18 @@ static bool apart(const void* a, size_t a_bytes, const void* b, size_t b_bytes) 
 
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
+// What awq_w4a16_rmsnorm_gemm uses: the GEMM's part, never smaller than the counter region, so a workspace
+// shared with awq_w4a16_gemm keeps its counters zero, then the normalised rows.
+static size_t rmsnorm_gemm_bytes(int64_t M, int64_t K, size_t gemm_bytes) {
+  return align256(std::max(gemm_bytes, (size_t)kCounterBytes)) + align256((size_t)M * (size_t)K * 2);
+}
+
 size_t awq_w4a16_rmsnorm_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t group_size,
                                               int32_t split_k, int32_t layout, int32_t act_dtype) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  // the GEMM's part is never smaller than the counter region, so a workspace shared with
-  // awq_w4a16_gemm keeps its counters zero
-  const size_t g = align256(std::max(awq_w4a16_gemm_workspace_bytes(M, N, K, group_size, split_k, layout),
-                                     (size_t)kCounterBytes));
-  const size_t xn = align256((size_t)M * (size_t)K * 2);
+  // BF16: the answer keeps the fp16 product [M, N] that earlier versions stored; the call needs no such part
   const size_t c16 = act_dtype == AWQ_DTYPE_BF16 ? align256((size_t)M * (size_t)N * 2) : 0;
-  return g + xn + c16;
+  return rmsnorm_gemm_bytes(M, K, awq_w4a16_gemm_workspace_bytes(M, N, K, group_size, split_k, layout)) + c16;
 }
 
 int awq_w4a16_rmsnorm_gemm(const void* x, int64_t ldx, const void* norm_w, float eps,
@@ -628,8 +630,7 @@ int awq_w4a16_rmsnorm_gemm(const void* x, int64_t ldx, const void* norm_w, float
   if (ldx < K || (ldx % 8) != 0 || (((uintptr_t)x) & 15)) return AWQ_ERR_STRIDE;
   if (ldc < N || (ldc % 8) != 0 || (((uintptr_t)c) & 15)) return AWQ_ERR_STRIDE;
   const size_t gws = awq_w4a16_gemm_workspace_bytes(M, N, K, group_size, split_k, layout);
-  if (workspace_bytes < awq_w4a16_rmsnorm_gemm_workspace_bytes(M, N, K, group_size, split_k, layout, act_dtype))
-    return AWQ_ERR_WORKSPACE;
+  if (workspace_bytes < rmsnorm_gemm_bytes(M, K, gws)) return AWQ_ERR_WORKSPACE;
   if ((((uintptr_t)workspace) & 255)) return AWQ_ERR_STRIDE;
   if (layout == AWQ_LAYOUT_DECODE_NARROW && scale_dtype == AWQ_DTYPE_F16 && M == 1 &&
       decode_covers(M, group_size) && (K % 32) == 0 && decode_narrow_bytes(K, N) <= 0x7FFFFFFFLL &&
@@ -658,13 +659,11 @@ int awq_w4a16_rmsnorm_gemm(const void* x, int64_t ldx, const void* norm_w, float
     if (launch_decode_narrow_norm(ga, qzeros != nullptr, (hipStream_t)stream)) return launch_status();
   }
   char* xn = (char*)workspace + align256(std::max(gws, (size_t)kCounterBytes));
-  const bool bf = act_dtype == AWQ_DTYPE_BF16;
-  if (bf && M > 65535) return AWQ_ERR_UNSUPPORTED;
   const int rc = awq_w4a16_rmsnorm(x, ldx, norm_w, eps, xn, K, M, K, act_dtype, norm_dtype, stream);
   if (rc != AWQ_OK) return rc;
   // bf16: the GEMM's epilogue converts its fp16 result (a launch over it took 2 us at 8 rows, 6 at 1000)
   return gemm_impl(xn, K, qweight, scales, qzeros, nullptr, c, ldc, M, N, K, group_size, split_k, layout, AWQ_DTYPE_F16,
-                   scale_dtype, AWQ_DTYPE_NONE, gws ? workspace : nullptr, gws, stream, 1, bf);
+                   scale_dtype, AWQ_DTYPE_NONE, gws ? workspace : nullptr, gws, stream, 1, act_dtype == AWQ_DTYPE_BF16);
 }
 
 }  // extern "C"

@@ -533,8 +533,8 @@ def rmsnorm_gemm(x: torch.Tensor, norm_w: torch.Tensor, eps: float, qweight: tor
         out = torch.empty((M, N), dtype=x.dtype, device=dev)
     else:
         check_out(out, M, N, x)
-    ws_bytes = int(lib.awq_w4a16_rmsnorm_gemm_workspace_bytes(M, N, K, int(group_size), int(split_k), lc,
-                                                              dtype_code(x.dtype)))
+    # the normalised rows are fp16 whatever x's dtype
+    ws_bytes = int(lib.awq_w4a16_rmsnorm_gemm_workspace_bytes(M, N, K, int(group_size), int(split_k), lc, L.DTYPE_F16))
     ws = WORKSPACE.get(dev, ws_bytes)
     rc = lib.awq_w4a16_rmsnorm_gemm(
         _ptr(x), K, _ptr(norm_w), float(eps), _ptr(qweight), _ptr(scales), _ptr(qzeros), _ptr(out),

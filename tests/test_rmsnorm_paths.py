@@ -59,3 +59,39 @@ def test_output_over_the_input_rows(M, off, dt):
     assert ops.rmsnorm_gemm(x, nw, 1e-6, *w, layout="autoawq", decode_layout="narrow", out=out).data_ptr() == out.data_ptr()
     # the narrow kernel's own norm and the row-norm launch give the same rows
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("M", [3, 100])
+def test_bf16_call_needs_no_room_for_its_product(M):
+    """The workspace of the fp16 call serves the bf16 one, to the byte."""
+    from litevllm_amd import _lib as L
+    from litevllm_amd import ops
+    K, N, G = 512, 264, 128
+    t = {k: torch.from_numpy(v).to(DEV) for k, v in make_awq_problem(M=M, K=K, N=N, group_size=G, seed=M).items()
+         if isinstance(v, np.ndarray)}
+    x, nw = t["x"].to(torch.bfloat16), torch.ones(K, dtype=torch.float16, device=DEV)
+    lib, qk = L.load(), ops.pack_decode_stream(t["qweight"])
+    need = int(lib.awq_w4a16_rmsnorm_gemm_workspace_bytes(M, N, K, G, 0, L.LAYOUT_DECODE_STREAM, L.DTYPE_F16))
+    ws = torch.zeros(need, dtype=torch.uint8, device=DEV)
+    out = torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
+    call = lambda nbytes: lib.awq_w4a16_rmsnorm_gemm(
+        x.data_ptr(), K, nw.data_ptr(), 1e-6, qk.data_ptr(), t["scales"].data_ptr(), t["qzeros"].data_ptr(), out.data_ptr(), N, M,
+        N, K, G, 0, L.LAYOUT_DECODE_STREAM, L.DTYPE_BF16, L.DTYPE_F16, L.DTYPE_F16, ws.data_ptr(), nbytes,
+        int(torch.cuda.current_stream().cuda_stream))
+    assert call(need - 1) == L.ERR_WORKSPACE
+    assert call(need) == 0
+    assert torch.equal(out, ops.rmsnorm_gemm(x, nw, 1e-6, t["qweight"], t["scales"], t["qzeros"], G, layout="autoawq",
+                                             decode_layout="stream" if M <= 32 else None))
+
+
+def test_bf16_rows_past_a_grid_dimension():
+    """More rows than a grid's y and z dimensions hold, as fp16 calls always took them."""
+    from litevllm_amd import ops
+    M, K, N, G = 65536 + 40, 64, 8, 32
+    t = {k: torch.from_numpy(v).to(DEV) for k, v in make_awq_problem(M=8, K=K, N=N, group_size=G, seed=1).items()
+         if isinstance(v, np.ndarray)}
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).to(DEV)
+    nw = torch.ones(K, dtype=torch.float16, device=DEV)
+    w = (t["qweight"], t["scales"], t["qzeros"], G)
+    y = ops.rmsnorm_gemm(x, nw, 1e-6, *w, layout="autoawq")
+    assert torch.equal(y, ops.gemm(ops.rmsnorm(x, nw, 1e-6), *w, layout="autoawq").to(torch.bfloat16))
