@@ -263,21 +263,26 @@ __global__ void __launch_bounds__(128 * NWN, 2) prefill_kn_kernel(const GemmArgs
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int row = wave_m * WM + mt * 16 + 4 * q + v;
-        cl[row * BN + c_chunk(row, cc >> 3) * 8 + (cc & 7)] = out_bits<T>(acc[mt][nt][v] + bv, p.c_bf16);
+        cl[row * BN + c_chunk(row, cc >> 3) * 8 + (cc & 7)] = to_bits<T>(acc[mt][nt][v] + bv);
       }
     }
   }
   __syncthreads();
   constexpr int CHUNKS = BM * CCH;
   static_assert(CHUNKS % NT == 0, "");
+  auto store = [&](auto via_bf16) {
 #pragma unroll
-  for (int j = 0; j < CHUNKS / NT; ++j) {
-    const int i = j * NT + tid;
-    const int row = i / CCH, ch = i % CCH;
-    const int grow = m0 + row, gcol = n0 + 8 * ch;
-    const u32x4 val = lds_all[row * CCH + c_chunk(row, ch)];
-    if (grow < p.M && gcol < p.N) *(u32x4*)(p.c + (int64_t)grow * p.ldc + gcol) = val;
-  }
+    for (int j = 0; j < CHUNKS / NT; ++j) {
+      const int i = j * NT + tid;
+      const int row = i / CCH, ch = i % CCH;
+      const int grow = m0 + row, gcol = n0 + 8 * ch;
+      u32x4 v = lds_all[row * CCH + c_chunk(row, ch)];
+      if constexpr (decltype(via_bf16)::value) v = via_bf16_words(v);
+      if (grow < p.M && gcol < p.N) *(u32x4*)(p.c + (int64_t)grow * p.ldc + gcol) = v;
+    }
+  };
+  if (std::is_same<T, f16>::value && p.c_bf16) store(std::true_type{});
+  else store(std::false_type{});
 }
 
 }  // namespace awq

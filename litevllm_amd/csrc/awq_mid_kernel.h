@@ -412,13 +412,14 @@ __global__ void __launch_bounds__(512, 2) mid_kernel(const GemmArgs p, const Mid
       b1 = load_bias(p.bias, p.bias_dtype, col + 1);
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) outl[(4 * rq + v) * 64 + 4 * c + P] = out_pack2<T>(o[0][v] + b0, o[1][v] + b1, p.c_bf16);
+    for (int v = 0; v < 4; ++v) outl[(4 * rq + v) * 64 + 4 * c + P] = pack2<T>(o[0][v] + b0, o[1][v] + b1);
   };
   auto write_out = [&](int mp, int nq) {
     __syncthreads();
     for (int i = tid; i < nq * 64; i += 512) {  // (row, word)
       const int row = i >> 4, c = i & 15, grow = m0 + 16 * mp + row, gword = t * 16 + c;
-      const u32x4 v = rd(lds0 + (uint32_t)(RED + row * 256 + c * 16));
+      u32x4 v = rd(lds0 + (uint32_t)(RED + row * 256 + c * 16));
+      if (std::is_same<T, f16>::value && p.c_bf16) v = via_bf16_words(v);
       if (grow < p.M && gword < NW) *(u32x4*)(p.c + (int64_t)grow * p.ldc + 8 * gword) = v;
     }
     __syncthreads();
@@ -532,12 +533,15 @@ __global__ void __launch_bounds__(256) mid_reduce_kernel(const GemmArgs p, const
       b1 = load_bias(p.bias, p.bias_dtype, col + 1);
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) outl[wave][v * 64 + 4 * c + P] = out_pack2<T>(o[0][v] + b0, o[1][v] + b1, p.c_bf16);
+    for (int v = 0; v < 4; ++v) outl[wave][v * 64 + 4 * c + P] = pack2<T>(o[0][v] + b0, o[1][v] + b1);
   }
   __syncthreads();
   const int grow = 4 * rq + P, gword = t * 16 + c;
-  if (on && grow < p.M && gword < (p.N >> 3))
-    *(u32x4*)(p.c + (int64_t)grow * p.ldc + 8 * gword) = *(const u32x4*)&outl[wave][P * 64 + 4 * c];
+  if (on && grow < p.M && gword < (p.N >> 3)) {
+    u32x4 v = *(const u32x4*)&outl[wave][P * 64 + 4 * c];
+    if (std::is_same<T, f16>::value && p.c_bf16) v = via_bf16_words(v);
+    *(u32x4*)(p.c + (int64_t)grow * p.ldc + 8 * gword) = v;
+  }
 }
 
 }  // namespace awq
