@@ -157,6 +157,20 @@ int awq_w4a16_gemm(const void* a, int64_t lda, const int32_t* qweight, const voi
                    int32_t act_dtype, int32_t scale_dtype, int32_t bias_dtype, void* workspace,
                    size_t workspace_bytes, void* stream);
 
+/* Kernel families of awq_w4a16_gemm. */
+#define AWQ_KERNEL_NARROW 1         /* decode, 16-column tiles (DECODE_NARROW) */
+#define AWQ_KERNEL_DECODE 2         /* decode, 128-column tiles */
+#define AWQ_KERNEL_DECODE_CHUNKS 3  /* the same in 32-row chunks */
+#define AWQ_KERNEL_MID 4            /* middle batches (DECODE_STREAM) */
+#define AWQ_KERNEL_PREFILL_STREAM 5 /* prefill (DECODE_STREAM) */
+#define AWQ_KERNEL_PREFILL 6        /* prefill (AUTOAWQ, KN_SEQ) */
+
+/* The family that serves such a call with a workspace of that many bytes (host only; 0 for sizes it
+ * refuses), and for AWQ_KERNEL_MID its plan: rows of a row tile and number of K ranges (each may be
+ * NULL; 0 for the others).  For tests and measurements: the choice may change between versions. */
+int awq_w4a16_gemm_kernel(int64_t M, int64_t N, int64_t K, int32_t group_size, int32_t split_k, int32_t layout,
+                          size_t workspace_bytes, int32_t* row_tile, int32_t* ranges);
+
 /* Allocation-free GEMM: awq_w4a16_gemm's computation, bit for bit, with its split-K counters and
  * partials in a fixed scratch array the library holds on every GPU it runs on (static device
  * memory, awq_w4a16_gemm_noalloc_max_workspace() bytes, kept until the process ends) instead of

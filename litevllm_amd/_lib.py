@@ -24,6 +24,13 @@ DTYPE_F16 = 1
 DTYPE_BF16 = 2
 DTYPE_F32 = 3
 
+KERNEL_NARROW = 1
+KERNEL_DECODE = 2
+KERNEL_DECODE_CHUNKS = 3
+KERNEL_MID = 4
+KERNEL_PREFILL_STREAM = 5
+KERNEL_PREFILL = 6
+
 OK = 0
 ERR_NULL = 1
 ERR_SHAPE = 2
@@ -60,6 +67,8 @@ SIGNATURES = {
     "awq_w4a16_gemm_rows_exact": (ctypes.c_int, [_c_p, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64,
                                                  _c_i64, _c_i64, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32,
                                                  _c_i32, _c_p, _c_sz, _c_p]),
+    "awq_w4a16_gemm_kernel": (ctypes.c_int, [_c_i64, _c_i64, _c_i64, _c_i32, _c_i32, _c_i32, _c_sz,
+                                             ctypes.POINTER(_c_i32), ctypes.POINTER(_c_i32)]),
     "awq_w4a16_gemm_noalloc_max_workspace": (_c_sz, []),
     "awq_w4a16_gemm_noalloc": (ctypes.c_int, [_c_p, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64,
                                               _c_i64, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_p]),

@@ -47,23 +47,56 @@ static bool decode_chunks(int64_t M, int64_t N, int64_t G) {
   return M > 32 && M <= 64 && decode_covers(32, G);
 }
 
+// Least rows (of 17 .. 32) from which the middle-batch kernel takes a call from the decode kernels.  Its blocks
+// cost 3 .. 4 us around their K loop, and in a K loop a group's scaling: so it is ahead where its K ranges
+// spread few tiles over the chip, in one round of whole-K blocks only from more rows on, in groups of 32 (a
+// scaling per k-step) only for small weights, and with more tiles than CUs hardly at all.  Measured on MI355X,
+// fp16 and bf16, K = 128 .. 14336, N = 256 .. 65536 (graph replays over rotated weights), decode against this
+// kernel, bf16, us:
+//   group 128: K = 4096 M = 25 N = 4096 12.0 -> 11.1, N = 24576 17.4 -> 17.3, N = 43008 30.2 -> 32.3 (M = 32
+//     33.6 -> 32.7); K = 2048 N = 24576 M = 25 11.2 -> 11.5, M = 28 11.7 -> 11.6; K = 1024 N = 4096 M = 25 7.8 -> 7.9
+//   group 64: K = 4096 N = 24576 M = 25 18.0 -> 19.2, M = 30 19.2 -> 19.3
+//   group 32: K = 4096 M = 25 N = 4096 13.3 -> 12.4, N = 6144 13.9 -> 14.6, N = 24576 22.4 -> 27.7; M = 17
+//     N = 4096 K = 2048 11.7 -> 10.7, K = 1024 8.6 -> 9.2
+// 17 rows at K <= 2048, else 25, is as far down as it goes: below, the decode kernels keep the call.
+static int64_t mid_least_rows(int64_t N, int64_t K, int64_t G) {
+  const int64_t tiles = cdiv(N, 128), cus = num_cus(), first = K <= 2048 ? 17 : 25, none = 33;
+  if (G == 32) return K >= 1536 && K <= 6144 && tiles * K <= 384 * cus ? first : none;
+  if (G == 64) return K < 1536 || tiles > cus ? none : 2 * tiles <= cus ? first : 30;
+  if (tiles > cus) return K < 2560 ? none : 31;
+  if (K < 1536) return 28;
+  return 2 * tiles <= cus || K > 2048 ? first : 28;
+}
+
 // Whether the middle-batch kernel (awq_mid_kernel.h) serves a call on the stream layout, and its plan:
 // "auto", or a forced split_k = 1 where auto's plan keeps the whole K per block (the same bits).
-// From 25 rows on, or 17 with K <= 2048 (against the decode kernels, fp16 / bf16: K = 2048, N = 2560 M = 17
-// 9.6 / 9.4 -> 8.1 / 8.3 us, but K = 4096, N = 24576 M = 17 17.6 / 15.7 -> 17.4 / 17.2 and M = 28
-// 18.6 / 18.0 -> 16.1 / 17.5); above 64, where its estimated time is an eighth below the prefill
-// kernel's (K = 4096, graph replays, start against this kernel: M = 128 N = 4096 29.0 -> 15.3 us,
+// From mid_least_rows on; above 64 rows where its estimated time is an eighth below the prefill
+// kernel's (K = 4096, graph replays, before this kernel and with it: M = 128 N = 4096 29.0 -> 15.3 us,
 // N = 24576 63.9 -> 33.1; M = 512 N = 4096 36.2 -> 20.9; M = 384 N = 24576 104 -> 84; at M = 512,
 // N = 24576, 100 - 108 against 103 us, the prefill kernel keeps the call).
 static bool mid_serves(int64_t M, int64_t N, int64_t K, int64_t G, int32_t split_k, int32_t layout, MidPlan* plan) {
-  if (layout != AWQ_LAYOUT_DECODE_STREAM || M <= (K <= 2048 ? 16 : 24) || split_k > 1) return false;
+  if (layout != AWQ_LAYOUT_DECODE_STREAM || M <= 16 || split_k > 1) return false;
   if (G < 32 || (G & (G - 1)) != 0 || (K % G) != 0 || (N % 8) != 0) return false;
-  // K <= 512 (at most one unit per share) stays with the decode kernels, which give the same bits on
-  // every layout: callers compare calls of this size across entry points
+  // K <= 512 stays with the decode kernels, which give the same bits there on the stream copy and on the
+  // AutoAWQ tensor (a call through one entry point may be compared with another's); 33 .. 64 rows in groups of
+  // 64 and 128 would run about 30% faster here (K = 512, N = 4096, M = 64 13.0 -> 7.7 us)
   if (M <= 64 && (K <= 512 || !decode_covers(M <= 32 ? M : 32, G))) return false;
+  if (M <= 32 && M < mid_least_rows(N, K, G)) return false;
   *plan = plan_mid(M, N, K, G);
   if (split_k == 1 && plan->splits != 1) return false;
   return M <= 64 || plan->us * 1.125 < prefill_us(M, N, K);
+}
+
+// The kernel family of a GEMM call (AWQ_KERNEL_*); `plan` is set for the middle-batch kernel.
+static int gemm_route(int64_t M, int64_t N, int64_t K, int64_t G, int32_t split_k, int32_t layout, int64_t rows,
+                      size_t workspace_bytes, MidPlan* plan) {
+  if (layout == AWQ_LAYOUT_DECODE_NARROW) return AWQ_KERNEL_NARROW;
+  // too small a workspace for the plan's K ranges: the decode kernels up to 64 rows, where it holds theirs
+  // (K < 1536: none), the prefill kernel above
+  if (rows <= 1 && mid_serves(M, N, K, G, split_k, layout, plan) && workspace_bytes >= plan->ws_bytes) return AWQ_KERNEL_MID;
+  if (decode_covers(M, G)) return AWQ_KERNEL_DECODE;
+  if (rows <= 1 && decode_chunks(M, N, G)) return AWQ_KERNEL_DECODE_CHUNKS;
+  return layout == AWQ_LAYOUT_DECODE_STREAM ? AWQ_KERNEL_PREFILL_STREAM : AWQ_KERNEL_PREFILL;
 }
 
 }  // namespace awq_host
@@ -236,23 +269,20 @@ static int gemm_impl(const void* a, int64_t lda, const int32_t* qweight, const v
   const bool seq = layout == AWQ_LAYOUT_KN_SEQ;
   const bool zp = qzeros != nullptr;
 
-  if (layout == AWQ_LAYOUT_DECODE_NARROW) {  // whole K per block: no workspace
+  MidPlan mp;
+  const bool aligned = workspace && !(((uintptr_t)workspace) & 15);
+  const int route = gemm_route(M, N, K, group_size, split_k, layout, rows, aligned ? workspace_bytes : 0, &mp);
+  if (route == AWQ_KERNEL_NARROW) {  // whole K per block: no workspace
     if (!launch_decode_narrow(ga, zp, act_dtype, scale_dtype, st)) return AWQ_ERR_UNSUPPORTED;
     return launch_status();
   }
-  MidPlan mp;
-  if (rows <= 1 && mid_serves(M, N, K, group_size, split_k, layout, &mp)) {
-    const bool held = workspace && workspace_bytes >= mp.ws_bytes && !(((uintptr_t)workspace) & 15);
-    if (mp.ws_bytes == 0 || held) {
-      ga.partial = mp.ws_bytes ? (float*)((char*)workspace + kCounterBytes) : nullptr;
-      ga.counters = (int*)workspace;
-      launch_mid(ga, mp, act_dtype, scale_dtype, st);
-      return launch_status();
-    }
-    // too small a workspace for the plan's K ranges: the decode kernels up to 64 rows, where it holds theirs
-    // (K < 1536: none), the prefill kernel above
+  if (route == AWQ_KERNEL_MID) {
+    ga.partial = mp.ws_bytes ? (float*)((char*)workspace + kCounterBytes) : nullptr;
+    ga.counters = (int*)workspace;
+    launch_mid(ga, mp, act_dtype, scale_dtype, st);
+    return launch_status();
   }
-  if (decode_covers(M, group_size)) {
+  if (route == AWQ_KERNEL_DECODE) {
     const DecodeMode mode = decode_mode(layout, act_dtype, scale_dtype);
     const DecodePlan sp = plan_decode(M, N, K, group_size, split_k, mode);
     if (sp.ws_bytes) {
@@ -267,7 +297,7 @@ static int gemm_impl(const void* a, int64_t lda, const int32_t* qweight, const v
     if (!launch_decode(ga, sp, mode, seq, zp, act_dtype, scale_dtype, st)) return AWQ_ERR_UNSUPPORTED;
     return launch_status();
   }
-  if (rows <= 1 && decode_chunks(M, N, group_size)) {
+  if (route == AWQ_KERNEL_DECODE_CHUNKS) {
     // 32-row chunks in order on the stream, sharing the workspace (each chunk's split-K
     // counters return to zero before the next starts)
     for (int64_t m0 = 0; m0 < M; m0 += 32) {
@@ -280,7 +310,7 @@ static int gemm_impl(const void* a, int64_t lda, const int32_t* qweight, const v
     return AWQ_OK;
   }
   if ((K % 32) != 0) return AWQ_ERR_SHAPE;
-  if (layout == AWQ_LAYOUT_DECODE_STREAM) {
+  if (route == AWQ_KERNEL_PREFILL_STREAM) {
     if (!launch_prefill_stream(ga, zp, act_dtype, scale_dtype, st)) return AWQ_ERR_UNSUPPORTED;
   } else if (!launch_prefill(ga, seq, zp, act_dtype, scale_dtype, st)) {
     return AWQ_ERR_UNSUPPORTED;
@@ -297,6 +327,16 @@ int awq_w4a16_gemm(const void* a, int64_t lda, const int32_t* qweight, const voi
                    size_t workspace_bytes, void* stream) {
   return gemm_impl(a, lda, qweight, scales, qzeros, bias, c, ldc, M, N, K, group_size, split_k, layout, act_dtype,
                    scale_dtype, bias_dtype, workspace, workspace_bytes, stream, 1);
+}
+
+int awq_w4a16_gemm_kernel(int64_t M, int64_t N, int64_t K, int32_t group_size, int32_t split_k, int32_t layout,
+                          size_t workspace_bytes, int32_t* row_tile, int32_t* ranges) {
+  if (M <= 0 || N <= 0 || K <= 0 || group_size <= 0 || split_k < 0 || (N % 8) != 0 || (K % group_size) != 0) return 0;
+  MidPlan mp{};
+  const int route = gemm_route(M, N, K, group_size, split_k, layout, 1, workspace_bytes, &mp);
+  if (row_tile) *row_tile = route == AWQ_KERNEL_MID ? 16 * mp.mt : 0;
+  if (ranges) *ranges = route == AWQ_KERNEL_MID ? mp.splits : 0;
+  return route;
 }
 
 size_t awq_w4a16_gemm_noalloc_max_workspace(void) { return kNoallocScratchBytes; }

@@ -134,3 +134,30 @@ def test_outlier_and_infinite_activations_in_groups_of_32(M, K, N, dt):
     assert np.array_equal(y[~fin], ye[~fin], equal_nan=True)
     ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(ye[fin]), 1.0))) - (10 if dt == torch.float16 else 7))
     assert (np.abs(y[fin] - ye[fin]) / ulp).max() <= 1.0
+
+
+# (M, K, N, G) on either side of the line from which 17 .. 32 rows leave the decode kernels
+DECODE_SIDE = [(17, 544, 256, 32), (20, 1024, 4096, 128), (27, 1280, 512, 128), (32, 1024, 264, 64), (32, 1024, 2560, 32),
+               (32, 2048, 6152, 32), (32, 4096, 3080, 32), (32, 8192, 136, 32), (29, 2048, 24576, 64), (27, 2048, 24576, 128),
+               (32, 2048, 32776, 128), (30, 2560, 34816, 128)]
+MID_SIDE = [(17, 1536, 264, 64), (17, 2048, 4096, 128), (28, 1280, 512, 128), (25, 4096, 3072, 32), (32, 2048, 6144, 32),
+            (30, 2048, 24576, 64), (28, 2048, 24576, 128), (31, 2560, 34816, 128), (33, 544, 256, 32)]
+
+
+@pytest.mark.parametrize("shape,mid", [(s, False) for s in DECODE_SIDE] + [(s, True) for s in MID_SIDE])
+def test_rows_from_which_the_kernel_takes_a_call(shape, mid):
+    """Each shape on the kernel that measured faster, and its outputs as test_mid_batch_vs_oracle holds them."""
+    from litevllm_amd import _lib as L
+    from litevllm_amd import ops
+    M, K, N, G = shape
+    print(f"mid or decode {shape}", flush=True)
+    ws = int(L.load().awq_w4a16_gemm_workspace_bytes(M, N, K, G, 0, L.LAYOUT_DECODE_STREAM))
+    route = L.load().awq_w4a16_gemm_kernel(M, N, K, G, 0, L.LAYOUT_DECODE_STREAM, ws, None, None)
+    assert route == (L.KERNEL_MID if mid else L.KERNEL_DECODE)
+    p = make_awq_problem(M=M, K=K, N=N, group_size=G, seed=M + K)
+    x = torch.from_numpy(p["x"]).to(torch.bfloat16)
+    w = tuple(torch.from_numpy(p[k]).to(DEV) for k in ("qweight", "scales", "qzeros")) + (G,)
+    y = ops.gemm(x.to(DEV), *w, layout="autoawq", decode_layout="stream" if M <= 32 else None).double().cpu().numpy()
+    ye = _expected(p, x, torch.from_numpy(p["scales"]), G, True, "bfloat16")
+    ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(ye), 1.0))) - 7)
+    assert (np.abs(y - ye) / ulp).max() <= 1.0
