@@ -117,9 +117,9 @@ int awq_w4a16_dequant(const int32_t* qweight, const void* scales, const int32_t*
 
 /* Workspace bytes awq_w4a16_gemm needs for these arguments (0 if none).  The workspace
  * starts with a fixed 64 KiB region of per-tile arrival counters followed by fp32 split-K
- * partials (the decode kernels', or the middle-batch kernel's K ranges; a call of the latter given
- * less than that runs on the decode kernels up to 64 rows, if it holds their partials, and on the
- * prefill kernel above).  The counter region must be zero the first time a workspace is used; every
+ * partials (the decode kernels', or the K ranges of the middle-batch or the prefill kernel; up to 64
+ * rows a call given less than that runs on the decode kernels, if it holds their partials, above on
+ * the middle-batch kernel, if it holds its partials, or else on whole-K prefill tiles).  The counter region must be zero the first time a workspace is used; every
  * call leaves it zero again, so a workspace allocated zeroed once can be reused by later
  * calls of any shape on the same stream.  Two calls that may run concurrently must not
  * share a workspace. */
@@ -166,8 +166,8 @@ int awq_w4a16_gemm(const void* a, int64_t lda, const int32_t* qweight, const voi
 #define AWQ_KERNEL_PREFILL 6        /* prefill (AUTOAWQ, KN_SEQ) */
 
 /* The family that serves such a call with a workspace of that many bytes (host only; 0 for sizes it
- * refuses), and for AWQ_KERNEL_MID its plan: rows of a row tile and number of K ranges (each may be
- * NULL; 0 for the others).  For tests and measurements: the choice may change between versions. */
+ * refuses), for AWQ_KERNEL_MID the rows of a row tile, and for it and AWQ_KERNEL_PREFILL_STREAM the
+ * number of K ranges (each may be NULL; 0 for the others).  For tests and measurements: the choice may change between versions. */
 int awq_w4a16_gemm_kernel(int64_t M, int64_t N, int64_t K, int32_t group_size, int32_t split_k, int32_t layout,
                           size_t workspace_bytes, int32_t* row_tile, int32_t* ranges);
 

@@ -87,10 +87,37 @@ static bool mid_serves(int64_t M, int64_t N, int64_t K, int64_t G, int32_t split
   return M <= 64 || plan->us * 1.125 < prefill_us(M, N, K);
 }
 
-// The kernel family of a GEMM call (AWQ_KERNEL_*); `plan` is set for the middle-batch kernel.
+// K ranges of the prefill stream kernel for a call on the stream layout ("auto" only), or 1.  The middle-batch
+// kernel took over most calls that had them; left are long K where its blocks, a row tile of up to 128 rows
+// each, make a second round (or, in groups of 32, scale at every k-step) and the prefill kernel's fewer, larger
+// tiles fit one.  Measured on MI355X, middle batch against ranges, us: M = 256 N = 16896 K = 12288 group 128
+// fp16 140 -> 118, bf16 152 -> 124; M = 512 N = 8192 K = 14336 group 32 bf16 172 -> 132; M = 1024 N = 4096
+// K = 12288 group 32 bf16 140 -> 117; below K = 6144 the middle-batch kernel wins as often as it loses.  The
+// factors are its measured over its estimated time, the mean of both types.
+static int range_serves(int64_t M, int64_t N, int64_t K, int64_t G, int32_t split_k, int32_t layout) {
+  if (layout != AWQ_LAYOUT_DECODE_STREAM || split_k != 0 || M <= 64 || K < 6144) return 1;
+  if (G < 32 || (G & (G - 1)) != 0 || (K % G) != 0 || (N % 8) != 0) return 1;
+  const int S = prefill_ranges(M, N, K);
+  if (S < 2) return 1;
+  const double us = prefill_ranges_us(M, N, K, S), mid = plan_mid(M, N, K, G).us * (G == 32 ? 1.16 : G == 64 ? 1.07 : 1.02);
+  return us < mid && us < prefill_us(M, N, K) ? S : 1;
+}
+// The partials go after the counter region, which a workspace shared between calls keeps zero.
+static size_t range_bytes(int64_t M, int64_t N, int S) {
+  return kCounterBytes + (size_t)S * (size_t)M * (size_t)N * sizeof(float);
+}
+
+// The kernel family of a GEMM call (AWQ_KERNEL_*); `plan` is set for the middle-batch kernel, `ranges` is the
+// prefill stream kernel's K ranges.
 static int gemm_route(int64_t M, int64_t N, int64_t K, int64_t G, int32_t split_k, int32_t layout, int64_t rows,
-                      size_t workspace_bytes, MidPlan* plan) {
+                      size_t workspace_bytes, MidPlan* plan, int* ranges) {
+  *ranges = 1;
   if (layout == AWQ_LAYOUT_DECODE_NARROW) return AWQ_KERNEL_NARROW;
+  const int S = rows <= 1 ? range_serves(M, N, K, G, split_k, layout) : 1;
+  if (S > 1 && workspace_bytes >= range_bytes(M, N, S)) {
+    *ranges = S;
+    return AWQ_KERNEL_PREFILL_STREAM;
+  }
   // too small a workspace for the plan's K ranges: the decode kernels up to 64 rows, where it holds theirs
   // (K < 1536: none), the prefill kernel above
   if (rows <= 1 && mid_serves(M, N, K, G, split_k, layout, plan) && workspace_bytes >= plan->ws_bytes) return AWQ_KERNEL_MID;
@@ -211,6 +238,8 @@ static size_t small_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t gro
 size_t awq_w4a16_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t group_size,
                                       int32_t split_k, int32_t layout) {
   if (M <= 0 || N <= 0 || K <= 0 || (N % 8) != 0 || split_k < 0) return 0;
+  const int S = group_size > 0 ? range_serves(M, N, K, group_size, split_k, layout) : 1;
+  if (S > 1) return range_bytes(M, N, S);
   MidPlan mp;
   if (mid_serves(M, N, K, group_size, split_k, layout, &mp)) return mp.ws_bytes;
   return decode_workspace_bytes(M, N, K, group_size, split_k, layout);
@@ -271,7 +300,8 @@ static int gemm_impl(const void* a, int64_t lda, const int32_t* qweight, const v
 
   MidPlan mp;
   const bool aligned = workspace && !(((uintptr_t)workspace) & 15);
-  const int route = gemm_route(M, N, K, group_size, split_k, layout, rows, aligned ? workspace_bytes : 0, &mp);
+  int ranges = 1;
+  const int route = gemm_route(M, N, K, group_size, split_k, layout, rows, aligned ? workspace_bytes : 0, &mp, &ranges);
   if (route == AWQ_KERNEL_NARROW) {  // whole K per block: no workspace
     if (!launch_decode_narrow(ga, zp, act_dtype, scale_dtype, st)) return AWQ_ERR_UNSUPPORTED;
     return launch_status();
@@ -311,6 +341,10 @@ static int gemm_impl(const void* a, int64_t lda, const int32_t* qweight, const v
   }
   if ((K % 32) != 0) return AWQ_ERR_SHAPE;
   if (route == AWQ_KERNEL_PREFILL_STREAM) {
+    if (ranges > 1) {
+      ga.partial = (float*)((char*)workspace + kCounterBytes);
+      ga.ksplit = ranges;
+    }
     if (!launch_prefill_stream(ga, zp, act_dtype, scale_dtype, st)) return AWQ_ERR_UNSUPPORTED;
   } else if (!launch_prefill(ga, seq, zp, act_dtype, scale_dtype, st)) {
     return AWQ_ERR_UNSUPPORTED;
@@ -333,9 +367,10 @@ int awq_w4a16_gemm_kernel(int64_t M, int64_t N, int64_t K, int32_t group_size, i
                           size_t workspace_bytes, int32_t* row_tile, int32_t* ranges) {
   if (M <= 0 || N <= 0 || K <= 0 || group_size <= 0 || split_k < 0 || (N % 8) != 0 || (K % group_size) != 0) return 0;
   MidPlan mp{};
-  const int route = gemm_route(M, N, K, group_size, split_k, layout, 1, workspace_bytes, &mp);
+  int S = 1;
+  const int route = gemm_route(M, N, K, group_size, split_k, layout, 1, workspace_bytes, &mp, &S);
   if (row_tile) *row_tile = route == AWQ_KERNEL_MID ? 16 * mp.mt : 0;
-  if (ranges) *ranges = route == AWQ_KERNEL_MID ? mp.splits : 0;
+  if (ranges) *ranges = route == AWQ_KERNEL_MID ? mp.splits : route == AWQ_KERNEL_PREFILL_STREAM ? S : 0;
   return route;
 }
 

@@ -279,6 +279,9 @@ struct GemmArgs {
   int norm_bf16;
   // fp16 kernels: the fp16 result is stored converted to bf16 (RMSNorm + GEMM of a bf16 tensor)
   int c_bf16;
+  // prefill stream kernel only: > 1 = K in that many ranges of whole stage pairs, each writing its fp32 sums to
+  // partial[range][M][N], added in range order by a second launch
+  int ksplit;
   // decode kernels only: > 1 = a row-exact launch (awq_w4a16_gemm_rows_exact) of that many grid
   // rows, M = 1: grid row y computes row y of the call as a lone M = 1 call would (row_slice)
   int rows;
