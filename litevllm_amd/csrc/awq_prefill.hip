@@ -503,12 +503,13 @@ static void launch_ps(const GemmArgs& a, int sbf, int log2g, hipStream_t st) {
   // Whole rounds of 256-column blocks, then a part round of them as 128-column blocks in a
   // second launch, where those fill the chip once: the part round runs at twice the blocks
   // for half the work each instead of leaving CUs idle (M = 2048, N = 12288: 384 blocks, 1.5
-  // rounds).  Also at row-tile counts that do not divide the CUs (K = 4096, one part round of
-  // 256-column blocks against this: M = 1500 N = 24576 316 -> 301 us, N = 22016 314 -> 298; M = 1700
-  // N = 28672 427 -> 406; M = 1200 N = 28672 313 -> 296).
+  // rounds).  Row-tile counts that do not divide the CUs take it from K = 512 on (one part round of
+  // 256-column blocks against this, fp16, K = 4096: M = 768 N = 28672 208 -> 191 us, M = 1280 N = 16896
+  // 209 -> 192, M = 1500 N = 22016 326 -> 311; over 30 shapes each, K = 512 even, K = 768 3% ahead, K = 256 2%
+  // behind, where a second launch costs more than the idle CUs: M = 768 N = 28672 27.9 -> 29.6).
   const int64_t full = (int64_t)tm * tn4 / cus * cus / tm;  // 256-column tiles of the whole rounds
   const int64_t rest = cdiv(a.N - full * 256, 128);
-  if (full > 0 && rest > 0 && tm * rest <= cus) {
+  if (full > 0 && rest > 0 && tm * rest <= cus && (cus % tm == 0 || a.K >= 512)) {
     wide((int)full, 0);
     narrow((int)rest, (int)full * 256);
     return;

@@ -27,3 +27,9 @@ def test_part_round_at_odd_row_tiles(M, K, N, G, dt):
     ye = x.double().cpu().numpy() @ w.astype(np.float64)
     ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(ye), 1.0))) - (10 if dt == torch.float16 else 7))
     assert (np.abs(y.double().cpu().numpy() - ye) / ulp).max() <= 1.0
+
+
+@pytest.mark.parametrize("K", [480, 512])
+def test_part_round_from_k_512_on(K):
+    """Both sides of the K from which such row-tile counts take the part round."""
+    test_part_round_at_odd_row_tiles(768, K, 23048, 32, torch.float16)
