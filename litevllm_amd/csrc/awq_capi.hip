@@ -711,9 +711,13 @@ int awq_w4a16_rmsnorm_gemm(const void* x, int64_t ldx, const void* norm_w, float
       decode_covers(M, group_size) && (K % 32) == 0 && decode_narrow_bytes(K, N) <= 0x7FFFFFFFLL &&
       M * ldx * 2 <= 0x7FFFFFFFLL && !(((uintptr_t)qweight) & 15) && !(((uintptr_t)scales) & 15) &&
       !(((uintptr_t)norm_w) & 15) && apart(c, (size_t)N * 2, x, (size_t)K * 2) &&
-      apart(c, (size_t)N * 2, norm_w, (size_t)K * 2)) {
+      apart(c, (size_t)N * 2, norm_w, (size_t)K * 2) &&
+      (act_dtype == AWQ_DTYPE_F16 || cdiv(N, 16) <= 2 * num_cus())) {
     // one launch: the narrow kernel normalises its staged rows itself.  Every block reads the whole row and
-    // the norm weights, so an output that lies over them takes the two launches below
+    // the norm weights, so an output that lies over them takes the two launches below.  A bf16 row does up to
+    // two tiles per CU: every block pays for the norm, and from the third on in further rounds (two launches
+    // against one, K = 1024 .. 20480: N = 8192 3 - 10% behind, N = 10240 2 - 28% ahead; K = 12288 N = 12288
+    // 20.4 against 25.9 us)
     GemmArgs ga{};
     ga.a = (const uint16_t*)x;
     ga.qw = (const uint32_t*)qweight;

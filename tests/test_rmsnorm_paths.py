@@ -95,3 +95,10 @@ def test_bf16_rows_past_a_grid_dimension():
     w = (t["qweight"], t["scales"], t["qzeros"], G)
     y = ops.rmsnorm_gemm(x, nw, 1e-6, *w, layout="autoawq")
     assert torch.equal(y, ops.gemm(ops.rmsnorm(x, nw, 1e-6), *w, layout="autoawq").to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("N", [8192, 8200, 10248])
+def test_one_bf16_row_on_either_side_of_two_tiles_per_cu(N):
+    """Up to two 16-column tiles per CU the narrow kernel normalises the row itself; the same bits as the row-norm
+    launch and the narrow GEMM on its row."""
+    test_bf16_rows_equal_converted_fp16_result(1, 512, N, 128, {"decode_layout": "narrow"})
