@@ -76,8 +76,8 @@ __device__ __forceinline__ uint16_t out_bits(float x, bool via_bf16) {
   return to_bits<T>(x);
 }
 // eight fp16 results converted to bf16 on their way from LDS to memory.  The kernels that store tiles convert
-// here, in a store loop of its own: next to the rounding, once per value, both forms are evaluated and one
-// selected, and a branch inside the loop keeps its LDS reads from overlapping (fp16 calls 0.9 us a prefill
+// here, under one branch for the tile: next to the rounding, once per value, both forms are evaluated and one
+// selected, and a branch at each 16 bytes keeps their LDS reads from overlapping (fp16 calls 0.9 us a prefill
 // block slower either way: M = 65, K = 256, N = 4096 9.7 -> 10.6 us)
 __device__ __forceinline__ u32x4 via_bf16_words(u32x4 v) {
 #pragma unroll

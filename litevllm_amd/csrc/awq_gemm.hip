@@ -270,19 +270,22 @@ __global__ void __launch_bounds__(128 * NWN, 2) prefill_kn_kernel(const GemmArgs
   __syncthreads();
   constexpr int CHUNKS = BM * CCH;
   static_assert(CHUNKS % NT == 0, "");
-  auto store = [&](auto via_bf16) {
+  // the whole share in registers, then one branch (a second store loop instead: fp16, K = 256, 2.7% slower)
+  u32x4 v[CHUNKS / NT];
 #pragma unroll
-    for (int j = 0; j < CHUNKS / NT; ++j) {
-      const int i = j * NT + tid;
-      const int row = i / CCH, ch = i % CCH;
-      const int grow = m0 + row, gcol = n0 + 8 * ch;
-      u32x4 v = lds_all[row * CCH + c_chunk(row, ch)];
-      if constexpr (decltype(via_bf16)::value) v = via_bf16_words(v);
-      if (grow < p.M && gcol < p.N) *(u32x4*)(p.c + (int64_t)grow * p.ldc + gcol) = v;
-    }
-  };
-  if (std::is_same<T, f16>::value && p.c_bf16) store(std::true_type{});
-  else store(std::false_type{});
+  for (int j = 0; j < CHUNKS / NT; ++j) {
+    const int i = j * NT + tid;
+    v[j] = lds_all[(i / CCH) * CCH + c_chunk(i / CCH, i % CCH)];
+  }
+  if (std::is_same<T, f16>::value && p.c_bf16)
+#pragma unroll
+    for (int j = 0; j < CHUNKS / NT; ++j) v[j] = via_bf16_words(v[j]);
+#pragma unroll
+  for (int j = 0; j < CHUNKS / NT; ++j) {
+    const int i = j * NT + tid;
+    const int grow = m0 + i / CCH, gcol = n0 + 8 * (i % CCH);
+    if (grow < p.M && gcol < p.N) *(u32x4*)(p.c + (int64_t)grow * p.ldc + gcol) = v[j];
+  }
 }
 
 }  // namespace awq
