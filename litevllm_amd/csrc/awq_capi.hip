@@ -309,7 +309,7 @@ static int gemm_impl(const void* a, int64_t lda, const int32_t* qweight, const v
   if (route == AWQ_KERNEL_MID) {
     ga.partial = mp.ws_bytes ? (float*)((char*)workspace + kCounterBytes) : nullptr;
     ga.counters = (int*)workspace;
-    launch_mid(ga, mp, act_dtype, scale_dtype, st);
+    if (!launch_mid(ga, mp, act_dtype, scale_dtype, st)) return AWQ_ERR_UNSUPPORTED;
     return launch_status();
   }
   if (route == AWQ_KERNEL_DECODE) {

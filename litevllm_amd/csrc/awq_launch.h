@@ -70,7 +70,8 @@ struct MidPlan {
   double us;
 };
 MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int64_t G);
-void launch_mid(const awq::GemmArgs& a, const MidPlan& m, int act, int sdt, hipStream_t st);
+// false: the plan has no kernel, nothing was launched.
+bool launch_mid(const awq::GemmArgs& a, const MidPlan& m, int act, int sdt, hipStream_t st);
 // Estimated time of the prefill stream kernel's launches for a call; its K ranges (1 = none), and their time.
 double prefill_us(int64_t M, int64_t N, int64_t K);
 int prefill_ranges(int64_t M, int64_t N, int64_t K);

@@ -42,23 +42,25 @@ MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int64_t G) {
 }
 
 template <typename T, bool FAST>
-static void launch_unr(const GemmArgs& a, int mt, const MidWork& wk, hipStream_t st) {
-  if (mt <= 2) launch_mid_g<2, true, T, FAST>(a, wk, st);
-  else if (mt == 3) launch_mid_g<3, true, T, FAST>(a, wk, st);
-  else launch_mid_g<4, true, T, FAST>(a, wk, st);
+static bool launch_unr(const GemmArgs& a, int mt, const MidWork& wk, hipStream_t st) {
+  if (mt <= 2) return launch_mid_g<2, true, T, FAST>(a, wk, st);
+  if (mt == 3) return launch_mid_g<3, true, T, FAST>(a, wk, st);
+  return launch_mid_g<4, true, T, FAST>(a, wk, st);
 }
 
-void launch_mid(const GemmArgs& a, const MidPlan& m, int act, int sdt, hipStream_t st) {
+bool launch_mid(const GemmArgs& a, const MidPlan& m, int act, int sdt, hipStream_t st) {
   const MidWork wk{m.tiles, m.splits, m.row_tiles, m.per, __builtin_ctz((unsigned)a.G), sdt == AWQ_DTYPE_BF16 ? 1 : 0};
-  if (a.M > 64) launch_mid_rounded(a, m.mt, wk, act, sdt, st);
-  else if (act == AWQ_DTYPE_F16 && sdt == AWQ_DTYPE_F16) launch_unr<f16, true>(a, m.mt, wk, st);
-  else if (act == AWQ_DTYPE_F16) launch_unr<f16, false>(a, m.mt, wk, st);
-  else launch_unr<bf16, false>(a, m.mt, wk, st);
-  if (a.M > 64 && m.splits > 1) {
+  bool done;
+  if (a.M > 64) done = launch_mid_rounded(a, m.mt, wk, act, sdt, st);
+  else if (act == AWQ_DTYPE_F16 && sdt == AWQ_DTYPE_F16) done = launch_unr<f16, true>(a, m.mt, wk, st);
+  else if (act == AWQ_DTYPE_F16) done = launch_unr<f16, false>(a, m.mt, wk, st);
+  else done = launch_unr<bf16, false>(a, m.mt, wk, st);
+  if (done && a.M > 64 && m.splits > 1) {
     const dim3 grid((unsigned)cdiv(cdiv(a.M, 4) * m.tiles, 4));
     if (act == AWQ_DTYPE_F16) hipLaunchKernelGGL((mid_reduce_kernel<f16>), grid, dim3(256), 0, st, a, wk);
     else hipLaunchKernelGGL((mid_reduce_kernel<bf16>), grid, dim3(256), 0, st, a, wk);
   }
+  return done;
 }
 
 }  // namespace awq_host

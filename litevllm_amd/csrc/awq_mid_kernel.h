@@ -551,14 +551,17 @@ using namespace awq;
 
 // Partials of a plan up to 64 rows: at most what the allocation-free entry point's scratch holds.
 constexpr size_t kMidPartialMax = (size_t)8 << 20;
-void launch_mid_rounded(const GemmArgs& a, int mt, const MidWork& wk, int act, int sdt, hipStream_t st);
+bool launch_mid_rounded(const GemmArgs& a, int mt, const MidWork& wk, int act, int sdt, hipStream_t st);
 
+// false: no such instantiation (eight row blocks leave no LDS for the constant sets of groups of 32)
 template <int MT, bool UNR, typename T, bool FAST>
-inline void launch_mid_g(const GemmArgs& a, const MidWork& wk, hipStream_t st) {
+inline bool launch_mid_g(const GemmArgs& a, const MidWork& wk, hipStream_t st) {
   const dim3 grid((unsigned)(wk.tiles * wk.splits * wk.row_tiles)), block(512);
   if (a.G >= 128) hipLaunchKernelGGL((mid_kernel<MT, UNR, T, FAST, 128>), grid, block, 0, st, a, wk);
   else if (a.G == 64) hipLaunchKernelGGL((mid_kernel<MT, UNR, T, FAST, 64>), grid, block, 0, st, a, wk);
   else if constexpr (mid_lds(MT, 32).r > 0) hipLaunchKernelGGL((mid_kernel<MT, UNR, T, FAST, 32>), grid, block, 0, st, a, wk);
+  else return false;
+  return true;
 }
 
 }  // namespace awq_host

@@ -275,3 +275,21 @@ def test_probe_read_rejects_bad_args_before_any_launch(lib):
     assert f(p, 64, 1, 96, 2, p, None) == L.ERR_SHAPE      # threads not a multiple of 64
     assert f(p, 64, 1, 2048, 2, p, None) == L.ERR_SHAPE
     assert f(p, 64, 1, 64, 3, p, None) == L.ERR_UNSUPPORTED
+
+
+def test_every_middle_batch_plan_has_a_kernel(lib):
+    """Row tiles of 32 to 128 rows; 128 in groups of 32 does not exist (its LDS) and is never planned.  (A plan
+    without a kernel would be refused, not skipped.)"""
+    import random
+    rng = random.Random(3)
+    tile = ctypes.c_int32()
+    seen = set()
+    for _ in range(4000):
+        G = rng.choice((32, 64, 128, 256))
+        M, N, K = round(17 * 2 ** (rng.random() * 7)), 8 * round(2 ** (rng.random() * 12)), G * rng.randint(1, 64)
+        ws = int(lib.awq_w4a16_gemm_workspace_bytes(M, N, K, G, 0, L.LAYOUT_DECODE_STREAM))
+        if lib.awq_w4a16_gemm_kernel(M, N, K, G, 0, L.LAYOUT_DECODE_STREAM, ws, tile, None) == L.KERNEL_MID:
+            seen.add((G == 32, tile.value))
+            assert tile.value % 16 == 0 and 32 <= tile.value <= (112 if G == 32 else 128), (M, N, K, G)
+            assert tile.value >= 64 or M <= 64
+    assert {t for _, t in seen} >= {32, 48, 64, 80, 96, 112, 128}
