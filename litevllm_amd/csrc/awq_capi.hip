@@ -61,7 +61,8 @@ static bool decode_chunks(int64_t M, int64_t N, int64_t G) {
 // 17 rows at K <= 2048, else 25, is as far down as it goes: below, the decode kernels keep the call.
 static int64_t mid_least_rows(int64_t N, int64_t K, int64_t G) {
   const int64_t tiles = cdiv(N, 128), cus = num_cus(), first = K <= 2048 ? 17 : 25, none = 33;
-  if (G == 32) return K >= 1536 && K <= 6144 && tiles * K <= 384 * cus ? first : none;
+  if (G == 32 && K < 1536) return K >= 1248 && 32 * tiles <= cus ? 25 : none;  // K = 1248 .. 1535: up to 8% ahead
+  if (G == 32) return K <= 6144 && tiles * K <= 384 * cus ? first : none;
   if (G == 64) return K < 1536 || tiles > cus ? none : 2 * tiles <= cus ? first : 30;
   if (tiles > cus) return K < 2560 ? none : 31;
   if (K < 1536) return 28;

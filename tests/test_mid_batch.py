@@ -137,10 +137,10 @@ def test_outlier_and_infinite_activations_in_groups_of_32(M, K, N, dt):
 
 
 # (M, K, N, G) on either side of the line from which 17 .. 32 rows leave the decode kernels
-DECODE_SIDE = [(17, 544, 256, 32), (20, 1024, 4096, 128), (27, 1280, 512, 128), (32, 1024, 264, 64), (32, 1024, 2560, 32),
+DECODE_SIDE = [(17, 544, 256, 32), (24, 1504, 512, 32), (32, 1504, 1032, 32), (20, 1024, 4096, 128), (27, 1280, 512, 128), (32, 1024, 264, 64), (32, 1024, 2560, 32),
                (32, 2048, 6152, 32), (32, 4096, 3080, 32), (32, 8192, 136, 32), (29, 2048, 24576, 64), (27, 2048, 24576, 128),
                (32, 2048, 32776, 128), (30, 2560, 34816, 128)]
-MID_SIDE = [(17, 1536, 264, 64), (17, 2048, 4096, 128), (28, 1280, 512, 128), (25, 4096, 3072, 32), (32, 2048, 6144, 32),
+MID_SIDE = [(17, 1536, 264, 64), (25, 1248, 1024, 32), (17, 2048, 4096, 128), (28, 1280, 512, 128), (25, 4096, 3072, 32), (32, 2048, 6144, 32),
             (30, 2048, 24576, 64), (28, 2048, 24576, 128), (31, 2560, 34816, 128), (33, 544, 256, 32)]
 
 
