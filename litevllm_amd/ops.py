@@ -69,9 +69,10 @@ def _require_device(*tensors: torch.Tensor | None) -> torch.device:
 
 def gemm_dims(qweight: torch.Tensor, layout: str) -> tuple[int, int]:
     """(K, N) of a packed weight in the given layout."""
+    # plain integers also while a caller is traced, when a shape holds tensors
     if layout == "ref":
-        return qweight.shape[1] * 8, qweight.shape[0]
-    return qweight.shape[0], qweight.shape[1] * 8
+        return int(qweight.shape[1]) * 8, int(qweight.shape[0])
+    return int(qweight.shape[0]), int(qweight.shape[1]) * 8
 
 
 # ------------------------------------------------------------------ dequant

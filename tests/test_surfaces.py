@@ -546,3 +546,19 @@ def test_out_argument_checked_before_launch():
     assert used and reason == "ok"
     ref = ops.gemm(x, *t, G)
     assert torch.equal(big[:, :N], ref) and bool((big[:, N:] == 0).all())
+
+
+@pytest.mark.parametrize("layout", ["autoawq", "ref"])
+def test_gemm_dims_are_integers_while_traced(layout):
+    """The library takes plain integers; under torch.jit.trace a shape's entries are tensors."""
+    import torch
+    from litevllm_amd import ops
+    seen = []
+
+    def call(qweight):
+        seen.append(ops.gemm_dims(qweight, layout))
+        return qweight + 1
+
+    torch.jit.trace(call, torch.zeros(64, 16, dtype=torch.int32), check_trace=False)
+    assert seen and all(type(v) is int for dims in seen for v in dims)
+    assert seen[0] == ((64, 128) if layout == "autoawq" else (128, 64))
