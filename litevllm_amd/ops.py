@@ -69,10 +69,11 @@ def _require_device(*tensors: torch.Tensor | None) -> torch.device:
 
 def gemm_dims(qweight: torch.Tensor, layout: str) -> tuple[int, int]:
     """(K, N) of a packed weight in the given layout."""
-    # plain integers also while a caller is traced, when a shape holds tensors
-    if layout == "ref":
-        return int(qweight.shape[1]) * 8, int(qweight.shape[0])
-    return int(qweight.shape[0]), int(qweight.shape[1]) * 8
+    shape = qweight.shape
+    rows, words = shape[0], shape[1]
+    if type(rows) is not int:  # while a caller is traced a shape holds tensors
+        rows, words = int(rows), int(words)
+    return (words * 8, rows) if layout == "ref" else (rows, words * 8)
 
 
 # ------------------------------------------------------------------ dequant
