@@ -163,10 +163,10 @@ def test_gemm_autoawq_vs_oracle(M, K, N, G, stream):
                                      (200, 512, 512, 32), (300, 2080, 520, 32)])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 def test_prefill_k_ranges(M, K, N, G, dt):
-    """Prefill calls whose 256 x 256 tiles cover at most half the CUs split K into ranges of
-    whole stage pairs (fp32 partials summed in range order by a second launch; the last range
-    of K % 64 == 32 ends on a half stage): within 1 ulp of the exact oracle on the fp16-rounded
-    weights, bias added once, bitwise reproducible."""
+    """Calls of 128 .. 384 rows over few columns, whose K is cut in ranges (the middle-batch kernel's:
+    fp32 partials summed in range order by a second launch; K % 64 == 32 ends on a half stage):
+    within 1 ulp of the exact oracle on the fp16-rounded weights, bias added once, bitwise
+    reproducible."""
     ops = _lib()
     _note(f"prefill k ranges M={M} K={K} N={N} G={G} {dt}")
     p = make_awq_problem(M=M, K=K, N=N, group_size=G, seed=M + K + G)

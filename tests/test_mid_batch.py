@@ -1,5 +1,5 @@
 """The middle-batch GEMM (17 rows to a few hundred, ``awq_mid_kernel.h``) through ``ops.gemm``, at the edges
-of its tiles: row tiles of 16 to 128 rows, a partial column tile, K that ends inside a stage, K ranges,
+of its tiles: row tiles of 32 to 128 rows, a partial column tile, K that ends inside a stage, K ranges,
 shares without work.  Every output within one ulp (of max(|y|, 1)) of the float64 product with the weights
 that the path multiplies: unrounded up to 64 rows, rounded once to the activation dtype above; bitwise
 the same on a second call."""
@@ -161,3 +161,34 @@ def test_rows_from_which_the_kernel_takes_a_call(shape, mid):
     ye = _expected(p, x, torch.from_numpy(p["scales"]), G, True, "bfloat16")
     ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(ye), 1.0))) - 7)
     assert (np.abs(y - ye) / ulp).max() <= 1.0
+
+
+# (M, K, N, G, rows of a row tile, K ranges): every instantiation above 64 rows, one row past the tile below where
+# that selects it, ragged columns, K that ends inside a stage or unit, several row tiles, K ranges
+ROW_TILES = [
+    (65, 544, 16656, 32, 80, 1), (65, 576, 16664, 64, 80, 1), (75, 640, 16776, 128, 80, 1), (200, 2080, 2752, 32, 80, 3),
+    (400, 4096, 520, 128, 80, 8), (81, 1056, 16656, 32, 96, 1), (96, 576, 16656, 64, 96, 1), (81, 768, 16664, 256, 96, 1),
+    (97, 1056, 16656, 32, 112, 1), (97, 1088, 16664, 64, 112, 1), (111, 1152, 16656, 128, 112, 1), (100, 4160, 5480, 32, 112, 5),
+    (113, 1088, 16656, 64, 128, 1), (128, 1152, 16664, 128, 128, 1), (113, 1280, 16656, 256, 128, 1), (120, 8192, 5480, 128, 128, 4)]
+
+
+@pytest.mark.parametrize("M,K,N,G,tile,ranges", ROW_TILES)
+def test_row_tiles_above_64_rows(M, K, N, G, tile, ranges):
+    import ctypes
+    from litevllm_amd import _lib as L
+    from litevllm_amd import ops
+    print(f"row tiles M={M} K={K} N={N} G={G} tile={tile} ranges={ranges}", flush=True)
+    t, r = ctypes.c_int32(), ctypes.c_int32()
+    ws = int(L.load().awq_w4a16_gemm_workspace_bytes(M, N, K, G, 0, L.LAYOUT_DECODE_STREAM))
+    assert L.load().awq_w4a16_gemm_kernel(M, N, K, G, 0, L.LAYOUT_DECODE_STREAM, ws, t, r) == L.KERNEL_MID
+    assert (t.value, r.value) == (tile, ranges)
+    p = make_awq_problem(M=M, K=K, N=N, group_size=G, seed=M + K)
+    qw, qz = (torch.from_numpy(p[k]).to(DEV) for k in ("qweight", "qzeros"))
+    for act, sdt in ((torch.float16, torch.float16), (torch.bfloat16, torch.float16), (torch.float16, torch.bfloat16)):
+        if sdt == torch.bfloat16 and K > 1200:  # the operand path alone: the short shapes do
+            continue
+        x, sc = torch.from_numpy(p["x"]).to(act), torch.from_numpy(p["scales"]).to(sdt)
+        y = ops.gemm(x.to(DEV), qw, sc.to(DEV), qz, G, layout="autoawq").double().cpu().numpy()
+        ye = _expected(p, x, sc, G, True, "float16" if act == torch.float16 else "bfloat16")
+        ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(ye), 1.0))) - (10 if act == torch.float16 else 7))
+        assert (np.abs(y - ye) / ulp).max() <= 1.0, (act, sdt)
