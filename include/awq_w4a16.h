@@ -62,9 +62,9 @@ extern "C" {
  * AWQ_LAYOUT_DECODE_STREAM : an AUTOAWQ qweight re-ordered by awq_w4a16_pack_decode_stream so
  *                      that the decode kernel reads it as contiguous 2 KiB runs; qzeros and
  *                      scales stay in the AUTOAWQ layout.  Accepted by awq_w4a16_gemm for every
- *                      M (K % 32 == 0): the decode kernel serves up to 16 or 24 rows with group
- *                      sizes 32/64/128, the middle-batch kernel up to a few hundred, the
- *                      prefill kernel the rest, so one copy serves all.
+ *                      M (K % 32 == 0): the decode kernel serves up to 16 rows with group sizes
+ *                      32/64/128, and up to 32 by shape, the middle-batch kernel up to a few
+ *                      hundred, the prefill kernel the rest, so one copy serves all.
  * AWQ_LAYOUT_DECODE_NARROW : an AUTOAWQ qweight re-ordered by awq_w4a16_pack_decode_narrow
  *                      into 16-column tiles cut along K into quads of four 32-row k-steps
  *                      (KQ = ceil(K / 128) quads per tile; k-steps past K are zero): the run of
@@ -141,12 +141,14 @@ size_t awq_w4a16_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t g
  *   bias: NULL or [N] of bias_dtype (F16, BF16 or F32), added once in fp32.
  *   c: [M, N] act_dtype, row stride ldc.
  *   split_k: number of contiguous K partitions of the decode kernel whose fp32 partial sums
- *            are added in a fixed order (0 = choose automatically; with 0 and the
- *            DECODE_STREAM layout the prefill kernel cuts K into 3 .. 8 ranges of whole
- *            64-row stage pairs where its 256 x 256 tiles cover at most a third of the CUs
- *            and the workspace holds their fp32 partials, summed in range order; otherwise
- *            the prefill kernel does not split K).  For a given (M, N, K, split_k) the result is bitwise
- *            reproducible.  Partition s covers rows [64 s I, min(64 (s+1) I, K)) with
+ *            are added in a fixed order (0 = choose automatically).  With 0 and the
+ *            DECODE_STREAM layout the middle-batch kernel cuts K into up to 16 ranges where its
+ *            tiles leave CUs idle, and the prefill kernel into 3 .. 8 ranges at K >= 6144 where
+ *            that is ahead, if the workspace holds their fp32 partials, summed in range order;
+ *            otherwise these kernels do not split K.  For a given (M, N, K, split_k), layout,
+ *            types and workspace size the result is bitwise reproducible; another layout, row
+ *            count or workspace may add the same products in another order.  Partition s of the
+ *            decode kernel covers rows [64 s I, min(64 (s+1) I, K)) with
  *            I = ceil(ceil(K / 64) / split_k), as in awq_fused_gemm.py:1798-1800.  The
  *            DECODE_NARROW layout never splits K (split_k is ignored there).
  *   Requirements: N % 8 == 0, group_size % 32 == 0, K % group_size == 0.
@@ -171,17 +173,17 @@ int awq_w4a16_gemm(const void* a, int64_t lda, const int32_t* qweight, const voi
 int awq_w4a16_gemm_kernel(int64_t M, int64_t N, int64_t K, int32_t group_size, int32_t split_k, int32_t layout,
                           size_t workspace_bytes, int32_t* row_tile, int32_t* ranges);
 
-/* Allocation-free GEMM: awq_w4a16_gemm's computation, bit for bit, with its split-K counters and
- * partials in a fixed scratch array the library holds on every GPU it runs on (static device
- * memory, awq_w4a16_gemm_noalloc_max_workspace() bytes, kept until the process ends) instead of
- * a caller's workspace.  No counterpart in the reference: it is for callers that cannot allocate
- * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc); it calls
- * no hipMalloc / hipFree or allocating routine.  Returns AWQ_ERR_WORKSPACE when the call would
- * need more workspace than that array holds (awq_w4a16_gemm_workspace_bytes of the same
- * arguments; the library's own split-K plans stay within it).  The first call on a device looks
- * the array up and clears its counters (a kernel on `stream`).  Every call on one GPU shares
- * that GPU's array: calls that may overlap on one GPU (other streams, other threads) race and
- * must be serialised by the caller. */
+/* Allocation-free GEMM: awq_w4a16_gemm's computation, up to 64 rows bit for bit (above, calls that
+ * would cut K into ranges run without them), with its split-K counters and partials in a fixed
+ * scratch array the library holds on every GPU it runs on (static device memory,
+ * awq_w4a16_gemm_noalloc_max_workspace() bytes, kept until the process ends) instead of a caller's
+ * workspace.  No counterpart in the reference: it is for callers that cannot allocate (code under
+ * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc); it calls no hipMalloc /
+ * hipFree or allocating routine.  Returns AWQ_ERR_WORKSPACE when the call would need more workspace
+ * than that array holds (awq_w4a16_gemm_workspace_bytes of the same arguments; the library's own
+ * split-K plans stay within it).  The first call on a device looks the array up and clears its
+ * counters (a kernel on `stream`).  Every call on one GPU shares that GPU's array: calls that may
+ * overlap on one GPU (other streams, other threads) race and must be serialised by the caller. */
 size_t awq_w4a16_gemm_noalloc_max_workspace(void);
 int awq_w4a16_gemm_noalloc(const void* a, int64_t lda, const int32_t* qweight, const void* scales,
                            const int32_t* qzeros, const void* bias, void* c, int64_t ldc, int64_t M, int64_t N,

@@ -533,8 +533,10 @@ inline void launch_t(const GemmArgs& a, const DecodePlan& s, hipStream_t st) {
     }
   }
   if constexpr (!ONE && STREAM) {
-    // the same with blocks of 4 waves, up to two tiles per CU (K = 4096, M = 8: N = 34816 23.6 -> 21.0 us, N =
-    // 65536 28.8 -> 26.4; at N = 81920 they trail, 37.5 -> 38.2)
+    // the same with blocks of 4 waves, up to two tiles per CU (K = 4096, fp16: N = 34816 M = 2 23.0 -> 20.0 us,
+    // M = 8 23.6 -> 21.2, M = 16 25.7 -> 24.3, M = 24 32.4 -> 30.4; N = 65536 M = 8 28.8 -> 26.3, M = 24 36.6 -> 34.0;
+    // over M = 2 .. 24, K = 1024 .. 8192, groups of 32 .. 128 and both types 10% ahead and nowhere behind; at
+    // M = 8, N = 81920 they trail, 37.5 -> 38.2)
     if (s.splits == 1 && s.tiles > num_cus() && s.tiles <= 2 * num_cus()) {
       launch_x<MT, SEQ, ZP, T, SBF, STREAM, ONE, false, 4>(a, s, 0, st);
       return;

@@ -7,13 +7,15 @@
 namespace awq_host {
 using namespace awq;
 
-// One block per CU; a block's time on MI355X is 2 us + 0.35 us per 16 rows outside its K loop
-// and 0.21 us + 0.08 us per 16 rows for each k-step of a share (128 k of the block), which
-// reproduces N = 24576, K = 4096 at one round of blocks (M = 32 / 48 / 64 / 80 / 96 / 128: 18.2 / 20.2 /
-// 22.3 / 24.5 / 28.7 / 33.1 us) to 5%.  K ranges add, up to 64 rows,
-// the hand-off (1.5 us) and one block's reading of its tile's partials (8 KB per range and 16 rows at
-// about 100 bytes a ns), above them the reduction launch (3 us) and the partials' round trip (about 6
-// TB/s).  Up to 64 rows there is one row tile;
+// One block per CU; a block's time on MI355X is 2 us + 0.35 us per 16 rows outside its K loop and 0.21 us +
+// 0.08 us per 16 rows for each k-step of a share (128 k of the block), which reproduces N = 24576, K = 4096
+// at one round of blocks (M = 32 / 48 / 64 / 80 / 96 / 128: 18.2 / 20.2 / 22.3 / 24.5 / 28.7 / 33.1 us) to
+// 5%: fp16 in groups of 128.  The measured time over this estimate, above 64 rows (means over K = 768 ..
+// 14336): groups of 128 0.93 .. 1.07 fp16, 1.06 .. 1.18 bf16; of 64 0.96 .. 1.10, 1.11 .. 1.23; of 32 1.06
+// .. 1.17, 1.16 .. 1.27.  The plan itself hardly depends on that factor, the choice of kernel does
+// (mid_least_rows, range_serves).  K ranges add, up to 64 rows, the hand-off (1.5 us) and one block's
+// reading of its tile's partials (8 KB per range and 16 rows at about 100 bytes a ns), above them the
+// reduction launch (3 us) and the partials' round trip (about 6 TB/s).  Up to 64 rows there is one row tile;
 // above, row tiles of 64 .. 128 rows: the plan with the least estimated time.
 MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int64_t G) {
   const int64_t tiles = cdiv(N, 128), cus = num_cus();

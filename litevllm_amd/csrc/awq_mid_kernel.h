@@ -26,8 +26,9 @@
 //    in range order.
 //  * The blocks of a column tile's row tiles are dispatched together on one XCD and read the
 //    tile's weights through its L2.
-//  * What bounds it: short calls, fixed costs (M = 64, N = K = 4096, 15.2 us: 1.3 us to the first operands,
-//    3.4 us of K loop, 2 us of final sum and partials, then the reduction launch); long loops, in about
+//  * What bounds it: short calls, fixed costs (M = 64, N = K = 4096, 14.6 us: 1.3 us to the first operands and
+//    3.4 us of K loop; the rest is the shares' sum, the partials and the last block's reading of them, the launch
+//    and its gap); long loops, in about
 //    equal parts and only partly overlapped, the MFMAs (M = 64: 0.27 us of a k-step's 0.5 us), the
 //    operand VALU and the DMA issue (8 rows x 128 bytes a request move 70 bytes a ns and CU, half of what
 //    linear requests do).  Tried: 32x32x16 MFMAs (5 VALU instructions per MFMA free instead of one, but
@@ -35,8 +36,8 @@
 //    issued at once: 3 - 15% slower; shares interleaved over K in 256-byte steps, against L2 channel
 //    conflicts: unchanged.
 //  * fp16, K = 4096, before (decode chunks of 32 rows, or 256-row prefill tiles cut in K ranges) and now:
-//    M = 57 N = 4096 23.8 -> 14.6 us, N = 24576 37.1 -> 22.3; M = 200 N = 6144 29.4 -> 19.4; M = 640
-//    N = 24576 207 -> 136; M = 256 K = 12288 N = 4096 48.4 -> 36.0.
+//    M = 57 N = 4096 24.3 -> 14.2 us, N = 24576 36.7 -> 21.6; M = 200 N = 6144 30.1 -> 20.7; M = 640
+//    N = 24576 204 -> 130; M = 256 K = 12288 N = 4096 50.9 -> 33.2.
 #pragma once
 
 #include "awq_common.h"

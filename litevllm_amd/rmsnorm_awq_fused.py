@@ -8,9 +8,10 @@ fp16 before the store, as in the reference (``rmsnorm_awq_fused.py:168-177``); f
 that fp16 result is converted to bf16.
 
 On the device this is ``awq_w4a16_rmsnorm_gemm``: one block per row reduces the row once and
-writes the normalised fp16 rows, then the dequant-GEMM kernels read them (the decode kernels
-for M <= 32, the MFMA prefill kernel above), instead of every output tile recomputing the
-row's sum of squares as the reference's kernel does.  The reference layout is converted once
+writes the normalised fp16 rows, then the dequant-GEMM kernels read them (decode, middle-batch
+or prefill, by shape) and convert a bf16 result as they store it, instead of every output tile
+recomputing the row's sum of squares as the reference's kernel does; a single row over few
+columns is normalised by the narrow decode kernel itself, in one launch.  The reference layout is converted once
 to the kernels' layout and cached on the weight, like every other entry point here.
 """
 from __future__ import annotations
